@@ -218,6 +218,16 @@ __device__ __forceinline__ uint64_t ballot(bool pred) { return __builtin_amdgcn_
 // Keep a wave-uniform value in a scalar register.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// LDS at byte address a.  The kernels that use it have no static LDS, so their
+// dynamic LDS starts at address 0 and a byte offset in it is its address; a
+// pointer made from the offset saves the add of that base (a constant 0 that
+// the compiler only learns after it has chosen the instructions).
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(3))) T* lds_ptr(uint32_t a) {
+  return reinterpret_cast<__attribute__((address_space(3))) T*>(a);
+}
+
 // A buffer resource over the n 4-byte elements at base + 4 first (wave-uniform
 // arguments, kept in scalar registers: a resource in vector registers makes
 // the compiler loop over the lanes' values).  Loads at byte offsets >= 4 n
@@ -1732,12 +1742,18 @@ constexpr int kDecThreads = kDecWaves * kLanes;
 constexpr int kEscWave = kDecWaves - 1;
 // per wave: index hash, status, escape nibbles
 constexpr int kDecPartBytes = (12 * kDecWaves + 15) / 16 * 16;
-// control words: [1] escape entries available (set when the reader stops),
-// [2 + b] steps of block parity b whose tables are not all in LDS (bit per
-// step, set by the mappers), [4 + b] block parity b has escapes and [6 + b]
-// escape entries consumed before block parity b (set by the coder)
-constexpr int kDecCtlBytes = 32;
+// control words: [0] stream words committed to the ring (set by the stream
+// wave after its last block), [1] escape entries available (set when the
+// reader stops), [2 + b] steps of block parity b whose tables are not all in
+// LDS (bit per step, set by the mappers); set by the coder: [4 + b] block
+// parity b has escapes, [6 + b] escape entries consumed and [8 + b] stream
+// words consumed before block parity b, for the last wave during that block,
+// [10 + b] the same entries for the mappers during the next block
+constexpr int kDecCtlBytes = 48;
 constexpr uint32_t kNoSym = 0xffffu;  // record of a lane past the chunk end
+// words after the stream ring that repeat its first ones: a step reads at most
+// kLanes words from a position below kRing, so its reads need no wrap
+constexpr int kRingMirror = 2 * kLanes;
 constexpr uint32_t kAllAvail = 0xffffffffu;
 
 struct DecArgs {
@@ -1771,49 +1787,46 @@ struct DecArgs {
 template <int SB>
 struct DecGeom {
   static constexpr int kPer = (SB + kMappers - 1) / kMappers;  // steps per mapper wave and block
-  static constexpr int kPfU32 = SB >= 16 ? 8 : 4;               // prefetch: u32 per lane
-  static constexpr int kPfWords = 2 * kPfU32 * kLanes;         // words per prefetch batch
-  static constexpr int kRing = SB >= 8 ? 2048 : 1024;          // stream ring (u16 words)
-  static constexpr int kLowWater = SB >= 8 ? 1024 : 512;
-  static constexpr int kPre = kLowWater / kPfWords;            // batches staged before block 0
-  static constexpr int kEscR = 2 * SB * kLanes;                // escape FIFO entries
-  static constexpr int kRingBytes = 2 * kRing;
-  static constexpr int kRecBytes = 2 * SB * kLanes * 8;
+  static constexpr int kBlockWords = SB * kLanes;      // a block's most words: one per lane and step
+  static constexpr int kPfU32 = kBlockWords / 2 / kLanes;  // stream batch: u32 per lane
+  static constexpr int kPfWords = kBlockWords;             // words per batch
+  static constexpr int kRing = 4 * kBlockWords;            // stream ring (u16 words)
+  static constexpr int kLowWater = 2 * kBlockWords;
+  static constexpr int kEscR = 2 * SB * kLanes;            // escape FIFO entries
+  static constexpr int kRingBytes = 2 * (kRing + kRingMirror);
+  static constexpr int kRecBytes = 2 * SB * kLanes * 4;
   static constexpr int kEscBytes = 4 * kEscR;
-  static constexpr int kMedBytes = 2 * SB * kLanes * 4;
-  // per step of two blocks: escaping lanes (u64) and the first entry's ordinal
-  static constexpr int kEscInfoBytes = 2 * SB * 16;
-  // [ring][records][escape FIFO][medians (latents)][escape steps][parts][control]
-  static constexpr int fixed(bool latents) {
-    return kRingBytes + kRecBytes + kEscBytes + (latents ? kMedBytes : 0) + kEscInfoBytes +
-           kDecPartBytes + kDecCtlBytes;
-  }
-  // a block start with fewer than kLowWater words buffered commits a batch:
-  // a batch covers one block's words (at most one per lane and step), so
-  // every block starts with at least SB * kLanes words buffered
-  static_assert(kLowWater >= SB * kLanes && kPfWords >= SB * kLanes &&
-                    kLowWater + kPfWords <= kRing && kPre >= 1 && kPfU32 <= kPfU32Max,
+  // [ring][records][escape FIFO][parts][control]
+  static constexpr int kFixed =
+      kRingBytes + kRecBytes + kEscBytes + kDecPartBytes + kDecCtlBytes;
+  // The stream wave commits during block j, knowing the position rp the block
+  // started at, batches until 2 kBlockWords past rp are buffered.  Block j
+  // reads at most kBlockWords from rp, so block j + 1 starts with at least as
+  // many buffered, and a commit ends below rp + 3 kBlockWords, so it never
+  // overwrites a word that block j may read.
+  static_assert(kLowWater + kPfWords <= kRing && kPfU32 <= kPfU32Max,
                 "decoder stream ring too small");
-  static_assert((kDecPartBytes + kDecCtlBytes) % 16 == 0, "LDS parts 16-byte aligned");
+  static_assert(kRingMirror == 2 * kLanes, "a batch's first u32 per lane is the mirror");
+  static_assert((kDecPartBytes + kDecCtlBytes) % 16 == 0 && kRingBytes % 16 == 0,
+                "LDS parts 16-byte aligned");
 };
 
-int dec_fixed_lds(bool latents, int sb) {
-  return sb >= 16 ? DecGeom<16>::fixed(latents)
-                  : (sb >= 8 ? DecGeom<8>::fixed(latents) : DecGeom<4>::fixed(latents));
+int dec_fixed_lds(int sb) {
+  return sb >= 16 ? DecGeom<16>::kFixed : (sb >= 8 ? DecGeom<8>::kFixed : DecGeom<4>::kFixed);
 }
 
-// Mapper record of one lane and step (8 bytes), tables in LDS when the step's
-// flag is 1:
-//   x: the lane's table | escape symbol << 16 (nsym - 1; kNoSym for a lane
-//      past the chunk end); the table is the LDS-local index times the
-//      lookup's bucket count (its first bucket: one add fewer per step for
-//      the coder), or the global index
-//   y: table offset
-// The coder overwrites x with the decoded value.
+// Mapper record of one lane and step (4 bytes), tables in LDS when the step's
+// flag is 1: the lane's table | escape symbol << 16 (nsym - 1; kNoSym for a
+// lane past the chunk end); the table is the LDS-local index times the
+// lookup's bucket count (its first bucket: one add fewer per step for the
+// coder), or the global index.  offset (the table's) stays with the mapper,
+// which stores the same lane and step later.  The coder overwrites the record
+// with the decoded symbol index.
 template <bool kImplicit, bool kWide>
-__device__ __forceinline__ uint2 dec_record(const DecArgs& a, const Tabs& tb, int lane, int t,
-                                            int len, int32_t start, int32_t in_b,
-                                            uint32_t& hash, uint32_t& status, bool& all_lds) {
+__device__ __forceinline__ uint32_t dec_record(const DecArgs& a, const Tabs& tb, int lane, int t,
+                                               int len, int32_t start, int32_t in_b,
+                                               uint32_t& hash, uint32_t& status, bool& all_lds,
+                                               uint32_t& offset) {
   const int p = lane + kLanes * t;
   const bool act = p < len;
   int32_t tbi =
@@ -1825,7 +1838,7 @@ __device__ __forceinline__ uint2 dec_record(const DecArgs& a, const Tabs& tb, in
   hash += ok ? index_term((uint32_t)p, (uint32_t)tbi) : 0u;
   const bool staged = (uint32_t)(tbi - tb.t_lo) < (uint32_t)tb.nt;
   all_lds = ballot(!staged) == 0;
-  uint32_t nsym, offset;
+  uint32_t nsym;
   if (all_lds) {  // separate loads per memory, as in dec_lookup
     const uint4 lm = tb.lmeta[tbi - tb.t_lo];
     nsym = lm.y;
@@ -1837,21 +1850,19 @@ __device__ __forceinline__ uint2 dec_record(const DecArgs& a, const Tabs& tb, in
     offset = (uint32_t)gm.offset;
     asm volatile("" : "+v"(nsym), "+v"(offset));
   }
-  uint2 r;
   constexpr int kB = kWide ? kWideBits : kLutBits;
-  r.x = (uint32_t)(all_lds ? (tbi - tb.t_lo) << kB : tbi) | ((act ? nsym - 1u : kNoSym) << 16);
-  r.y = offset;
-  return r;
+  return (uint32_t)(all_lds ? (tbi - tb.t_lo) << kB : tbi) | ((act ? nsym - 1u : kNoSym) << 16);
 }
 
-// Mapper record with the search lookups (all tables in LDS): x = the table's
-// first segment (table * kSearchEntries, below 2^16 when the blob has the
-// search lookups) | starts index of its escape symbol << 16 (kNoSym past the
-// chunk end), y = offset - the starts index of its symbol 0, so that the
-// decoded starts index + y is the value.
-__device__ __forceinline__ uint2 dec_record_search(const DecArgs& a, const Tabs& tb, int lane,
-                                                   int t, int len, int32_t in_b, uint32_t& hash,
-                                                   uint32_t& status) {
+// Mapper record with the search lookups (all tables in LDS): the table's first
+// segment (table * kSearchEntries, below 2^16 when the blob has the search
+// lookups) | starts index of its escape symbol << 16 (kNoSym past the chunk
+// end).  The coder's symbol is a starts index: offset is the table's less the
+// starts index of its symbol 0 (first).
+__device__ __forceinline__ uint32_t dec_record_search(const DecArgs& a, const Tabs& tb, int lane,
+                                                      int t, int len, int32_t in_b,
+                                                      uint32_t& hash, uint32_t& status,
+                                                      uint32_t& offset, uint32_t& first) {
   const int p = lane + kLanes * t;
   const bool act = p < len;
   int32_t tbi = in_b;
@@ -1861,11 +1872,9 @@ __device__ __forceinline__ uint2 dec_record_search(const DecArgs& a, const Tabs&
   tbi = ok ? tbi : 0;
   hash += ok ? index_term((uint32_t)p, (uint32_t)tbi) : 0u;
   const uint4 lm = tb.lmeta[tbi];
-  uint2 r;
-  const uint32_t first = lm.x + (uint32_t)(kStartsTablePad * tbi);  // starts index of symbol 0
-  r.x = (uint32_t)tbi * (uint32_t)kSearchEntries | ((act ? first + lm.y - 1u : kNoSym) << 16);
-  r.y = lm.z - first;
-  return r;
+  first = lm.x + (uint32_t)(kStartsTablePad * tbi);  // starts index of symbol 0
+  offset = lm.z;
+  return (uint32_t)tbi * (uint32_t)kSearchEntries | ((act ? first + lm.y - 1u : kNoSym) << 16);
 }
 
 // One level down from a dense lookup entry e: entry i of its sub-block (LDS
@@ -1885,7 +1894,9 @@ __device__ __forceinline__ uint64_t sub_entry(const Tabs& tb, uint64_t e, uint32
   return r;
 }
 
-__device__ __forceinline__ bool dense_entry(uint64_t e) { return (uint32_t)(e >> 48) == 0xffffu; }
+__device__ __forceinline__ bool dense_entry(uint64_t e) {
+  return (uint32_t)(e >> 32) >= 0xffff0000u;
+}
 
 // (symbol, start, freq) from a lookup entry with at most one other start
 // (see the blob layout): s or s + 1.
@@ -1904,38 +1915,31 @@ __device__ __forceinline__ void lut_pick(uint64_t e, uint32_t cum, uint32_t& s, 
 // of its sub-block, for a dense sub-range the exact entry of value cum & 15
 // (see the blob layout).  kWide: the wide lookups, bucket cum >> 5 and, for
 // a dense bucket, sub-range (cum >> 1) & 15 of its sub-block.  t is the
-// staged table's first bucket (kLds) or the global table index.  kEarly: the
-// entry is decoded before the dense test's branch (the asm keeps it there)
-// and a dense lane's values are redone from the entry one or two levels
-// down, which overlaps the branch's latency with that work (512x768 decode
-// 23.6 -> 23.2 us with one workgroup per CU); else after it, which spends
-// no issue slots on the redone work (batch-64 skew decode 95.9 -> 93.9 us
-// with three per CU).
-template <bool kLds, bool kWide = false, bool kEarly = false>
+// staged table's first bucket (kLds) or the global table index.
+template <bool kLds, bool kWide>
+__device__ __forceinline__ uint64_t dense_lookup(const Tabs& tb, uint64_t e, uint32_t cum,
+                                                 bool dense) {
+  if constexpr (kWide) {
+    // a wide bucket's sub-ranges (two values) are never dense
+    if (dense) e = sub_entry<kLds>(tb, e, (cum >> kWideSubShift) & (kSubSize - 1));
+  } else {
+    if (dense) e = sub_entry<kLds>(tb, e, (cum >> kSubBits) & (kSubSize - 1));
+    const bool dense3 = dense & dense_entry(e);
+    if (__builtin_expect(ballot(dense3) != 0ull, 0) && dense3)
+      e = sub_entry<kLds>(tb, e, cum & (kSubSize - 1));
+  }
+  return e;
+}
+
+template <bool kLds, bool kWide = false>
 __device__ __forceinline__ void dec_lookup(const Tabs& tb, uint32_t t, uint32_t cum, bool act,
                                            uint32_t& s, uint32_t& st, uint32_t& fr) {
   constexpr int kB = kWide ? kWideBits : kLutBits;
   const uint32_t li = (kLds ? t : t << kB) + (cum >> (16 - kB));
   uint64_t e = kLds ? tb.llut[li] : tb.glut[li];
-  if (kEarly) {
-    lut_pick(e, cum, s, st, fr);
-    asm volatile("" : "+v"(s), "+v"(st), "+v"(fr));
-  }
-  const uint64_t dm = ballot(act & dense_entry(e));
-  if (!kEarly) asm volatile("" ::"s"(dm));
-  if (__builtin_expect(dm != 0ull, 0)) {
-    if constexpr (kWide) {
-      // a wide bucket's sub-ranges (two values) are never dense
-      if (act & dense_entry(e)) e = sub_entry<kLds>(tb, e, (cum >> kWideSubShift) & (kSubSize - 1));
-    } else {
-      if (act & dense_entry(e)) e = sub_entry<kLds>(tb, e, (cum >> kSubBits) & (kSubSize - 1));
-      const uint64_t dm3 = ballot(act & dense_entry(e));
-      if (__builtin_expect(dm3 != 0ull, 0) && (act & dense_entry(e)))
-        e = sub_entry<kLds>(tb, e, cum & (kSubSize - 1));
-    }
-    if (kEarly) lut_pick(e, cum, s, st, fr);
-  }
-  if (!kEarly) lut_pick(e, cum, s, st, fr);
+  const bool dense = act & dense_entry(e);
+  if (__builtin_expect(ballot(dense) != 0ull, 0)) e = dense_lookup<kLds, kWide>(tb, e, cum, dense);
+  lut_pick(e, cum, s, st, fr);
 }
 
 // cum -> (symbol, start, freq) with the search lookups, all tables in LDS;
@@ -2102,19 +2106,17 @@ __device__ __forceinline__ void stage_late(Tabs& T, const EarlyStage& e, uint4* 
   __syncthreads();
 }
 
-// Word stream of one chunk: prefetched from HBM into registers (kPfWords words
-// ahead) and copied into an LDS ring of kRing words holding the words
-// [rp, filled) (positions mod kRing), kPfWords words at a time.  At the start
-// of every block the coder commits the batch prefetched into registers (pf,
-// words [filled, filled + kPfWords)) when fewer than kLowWater words are
-// buffered, then prefetches the next batch.  This is the only place pf is
-// loaded, so the loads stay in flight between blocks.  A step refills at most
-// one word per lane, and a block starts with at least SB * kLanes buffered
-// words, so refills need no check.
+// Word stream of one unit: prefetched from HBM into registers (one batch of
+// kPfWords words ahead) and copied into an LDS ring of kRing words, by the
+// workgroup's last wave (the escape reader, idle otherwise), so that none of
+// it is on the coder's chain.  The ring holds words up to `filled` (positions
+// mod kRing); the coder publishes its position rp at each block start.  pf
+// (words [filled, filled + kPfWords)) is loaded right after the batch before
+// it was committed, a block or more before its own commit.
 struct Stream {
   const uint32_t* __restrict__ s32;
   uint32_t lane_off;  // 4 * lane: the loads' only per-lane operand
-  int q, q32, rp, filled;
+  int q, q32, filled;
   uint32_t pf[kPfU32Max];  // the first DecGeom<SB>::kPfU32 in use
 };
 
@@ -2144,48 +2146,44 @@ __device__ __forceinline__ void stream_batch32(const Stream& S, int i32, uint32_
     out[kk] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)(S.lane_off + 4u * kLanes * kk), 0, 0);
 }
 
-// Block start: commit pf if needed, then fetch the next batch.
+// Batch pf -> ring, then the next batch's loads.
 template <int SB>
-__device__ __forceinline__ void stream_block_start(Stream& S, uint32_t* ring32, int lane) {
+__device__ __forceinline__ void stream_commit(Stream& S, uint32_t* ring32, int lane) {
   using G = DecGeom<SB>;
-  const bool commit = S.filled - S.rp < G::kLowWater && S.filled < S.q;
-  if (commit) {
-    // a batch starts at a multiple of its size in the ring, which holds a
-    // whole number of batches: it never wraps, one mask for all its words
-    static_assert((G::kRing / 2) % (G::kPfWords / 2) == 0, "ring of whole batches");
-    uint32_t* dst = ring32 + (((uint32_t)S.filled >> 1) & (G::kRing / 2 - 1)) + lane;
+  // a batch starts at a multiple of its size in the ring, which holds a
+  // whole number of batches: it never wraps, one mask for all its words
+  static_assert(G::kRing % G::kPfWords == 0, "ring of whole batches");
+  const uint32_t at = ((uint32_t)S.filled >> 1) & (G::kRing / 2 - 1);
+  uint32_t* dst = ring32 + at + lane;
 #pragma unroll
-    for (int kk = 0; kk < G::kPfU32; ++kk) dst[kk * kLanes] = S.pf[kk];
-    S.filled = uni(S.filled + G::kPfWords);
-    stream_batch32<G::kPfU32>(S, S.filled >> 1, S.pf);
-  }
+  for (int kk = 0; kk < G::kPfU32; ++kk) dst[kk * kLanes] = S.pf[kk];
+  // the mirror (of a batch at the ring's start; else its words once more)
+  ring32[(at ? at : (uint32_t)(G::kRing / 2)) + lane] = S.pf[0];
+  S.filled = uni(S.filled + G::kPfWords);
+  stream_batch32<G::kPfU32>(S, S.filled >> 1, S.pf);
 }
 
-// A refill past the stream end reads stale ring words; the chunk is then
-// marked corrupt by the final check that exactly the stream was consumed.
-// Every lane reads (the lane's rank among the refilling lanes, counted on top
-// of the stream position by mbcnt's accumulator) and only refilling lanes
-// keep the word (the read's value is opaque to the compiler, so the select
-// is not turned into an exec-masked branch around it).  kSkip: the read is
-// skipped when no lane refills (a uniform branch on the compare).  Measured
-// on MI355X: with one workgroup per CU, where the step's latency bounds the
-// launch, the branch lengthens the step (2160x3840 latent 231 -> 238 us,
-// 512x768 23.8 -> 24.4 us); with several per CU, where issue slots do, it
-// saves them (batch-64 skew 101 -> 95 us, uniform 95 -> 90 us).
-template <int SB, bool kSkip>
-__device__ __forceinline__ void dec_refill(bool need, uint32_t& x, Stream& S, const uint16_t* ring,
-                                           int lane) {
+// During a block that starts at stream position rp (see DecGeom).
+template <int SB>
+__device__ __forceinline__ void stream_block(Stream& S, int rp, uint32_t* ring32, int lane) {
+  while (S.filled - rp < DecGeom<SB>::kLowWater && S.filled < S.q)
+    stream_commit<SB>(S, ring32, lane);
+}
+
+// Refill of a step.  A refill past the stream end reads stale ring words; the
+// unit is then marked corrupt by the final check that exactly the stream was
+// consumed.  Every lane reads (the lane's rank among the refilling lanes,
+// counted on top of the stream position by mbcnt's accumulator) and only
+// refilling lanes keep the word, by the byte selector of one v_perm_b32.
+template <int SB>
+__device__ __forceinline__ void dec_refill(bool need, uint32_t& x, int& rp) {
   const uint64_t m = ballot(need);
-  if (!kSkip || m != 0ull) {
-    // the ring position (< kRing) plus the rank: past the end it reads the
-    // mirrored first words
-    const uint32_t pos = __builtin_amdgcn_mbcnt_hi(
-        (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)S.rp));
-    uint32_t w = ring[pos & (DecGeom<SB>::kRing - 1)];
-    asm volatile("" : "+v"(w));
-    x = need ? ((x << 16) | w) : x;
-    S.rp += __popcll(m);
-  }
+  const uint32_t pos = __builtin_amdgcn_mbcnt_hi(
+      (uint32_t)(m >> 32),
+      __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)rp & (uint32_t)(DecGeom<SB>::kRing - 1)));
+  const uint32_t w = *lds_ptr<uint16_t>(pos << 1);
+  x = __builtin_amdgcn_perm(x, w, need ? 0x05040100u : 0x07060504u);
+  rp += __popcll(m);
 }
 
 // Escape section of one chunk, read from the chunk's end: escape u32 m holds
@@ -2310,32 +2308,232 @@ __device__ __forceinline__ void esc_resolve(uint64_t em, uint32_t base, uint32_t
   enib += e ? (raw ? ((31u - (uint32_t)__clz((int)raw)) >> 2) + 2u : 1u) : 0u;
 }
 
-// One decode step of the coder wave; returns the decoded value and, in em,
-// the lanes that decoded the escape bin (their values are resolved by the
-// mappers, off the state chain).  kFull: every lane is active and no offset
-// can overflow with a symbol index.
-template <bool kLds, bool kFull, int SB, bool kSearch = false, bool kWide = false,
-          bool kSkip = false>
-__device__ __forceinline__ uint32_t dec_step(const Tabs& tb, const uint2 r, uint32_t& x,
-                                             Stream& S, const uint16_t* ring, uint64_t& em,
-                                             uint32_t& status, int lane) {
-  const uint32_t es = r.x >> 16;
+// One decode step of the coder wave; returns the word that replaces the record:
+// the decoded symbol index | the block's escapes before this step << 16 (esc,
+// the same in every lane, which counts this step's in; their values are
+// resolved by the mappers, off the state chain).  kFull: every lane is active.
+template <bool kLds, bool kFull, int SB, bool kSearch = false, bool kWide = false>
+__device__ __forceinline__ uint32_t dec_step(const Tabs& tb, const uint32_t r, uint32_t& x,
+                                             int& rp, uint32_t& esc) {
+  const uint32_t es = r >> 16;
   const bool act = kFull || es != kNoSym;
   const uint32_t cum = x & 0xffffu;
   uint32_t s, st, fr;
-  if constexpr (kSearch) dec_lookup_search(tb, r.x & 0xffffu, cum, act, s, st, fr);
-  else dec_lookup<kLds, kWide, !kSkip>(tb, r.x & 0xffffu, cum, act, s, st, fr);
+  if constexpr (kSearch) dec_lookup_search(tb, r & 0xffffu, cum, act, s, st, fr);
+  else dec_lookup<kLds, kWide>(tb, r & 0xffffu, cum, act, s, st, fr);
   const uint32_t xn = __umul24(fr, x >> 16) + cum - st;
   x = act ? xn : x;
-  dec_refill<SB, kSkip>(act & (x < kStateLow), x, S, ring, lane);
-  // value + offset for an ordinary symbol: s < 2^16, so the int32 sum overflows
-  // exactly when it wraps below the offset
-  const int32_t o = (int32_t)(s + r.y);
-  const bool esc = act & (s == es);
-  em = ballot(esc);
-  const bool oob = act & !esc & !kFull & (o < (int32_t)r.y);
-  status |= oob ? GAANS_ST_CORRUPT : 0u;
-  return (uint32_t)(oob ? 0 : o);
+  dec_refill<SB>(act & (x < kStateLow), x, rp);
+  const uint32_t word = s | (esc << 16);
+  esc += (uint32_t)__popcll(ballot(act & (s == es)));
+  return word;
+}
+
+// State update and refill rank of a step, from lookup entry (lo, hi), with at
+// most one other start in its range (s or s + 1, "up"), and the state x.
+//   up:  x' = freq1 xh + cum - st1,  freq1 = (hi >> 16) + 1, st1 = (lo >> 16) + 1
+//   not: x' = freq0 xh + cum - st0,  freq0 = st1 - st0
+// (xh = x >> 16), both written as F H + (pre - (st1 - 1) - up) with F = freq -
+// 1, H = xh + 1 - up and pre = xh + cum: no select of the starts, and xh + 1
+// and pre are ready before the entry is.  F <= 65535 and H <= 65536, so the
+// product is a 24-bit multiply-add.  Then the lanes with x' < 2^16 (m) refill,
+// and pos is twice the lane's rank among them on top of the ring position at.
+// tbase is the byte offset of the next step's first bucket, from its record.
+//
+// One asm block: the 13 operations between the two LDS reads are the step's
+// chain, at one issue per four cycles each, and the compiler spends 22 on them
+// (unpacked fields, two selects, a 64-bit dense test and its branch).  It
+// keeps two other operations between a vector compare and a reader of its mask
+// (CDNA3's wait states): up and tbase, which nothing waits for, fill one pair.
+struct StepUpdate {
+  uint32_t xn, up, pos, tbase;
+  uint64_t m;
+};
+
+__device__ __forceinline__ StepUpdate step_update(uint32_t lo, uint32_t hi, uint32_t x,
+                                                  uint32_t at, uint32_t next_rec) {
+  StepUpdate u;
+  const uint32_t xh1 = (x >> 16) + 1u, pre = (x >> 16) + (x & 0xffffu);
+  uint32_t f, h, t;
+  uint64_t unused;
+  register uint64_t m asm("vcc");
+  asm("v_cmp_gt_u32_sdwa vcc, %[x], %[lo] src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+      "v_sub_u32_sdwa %[f], %[lo], %[lo] dst_sel:DWORD dst_unused:UNUSED_PAD "
+      "src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+      "v_sub_u32_sdwa %[t], %[pre], %[lo] dst_sel:DWORD dst_unused:UNUSED_PAD "
+      "src0_sel:DWORD src1_sel:WORD_1\n\t"
+      "v_subbrev_co_u32_e64 %[h], %[un], 0, %[xh1], vcc\n\t"
+      "v_cndmask_b32_sdwa %[f], %[f], %[hi], vcc dst_sel:DWORD dst_unused:UNUSED_PAD "
+      "src0_sel:DWORD src1_sel:WORD_1\n\t"
+      "v_subbrev_co_u32_e64 %[t], %[un], 0, %[t], vcc\n\t"
+      "v_mad_u32_u24 %[xn], %[f], %[h], %[t]\n\t"
+      "v_cmp_gt_u32_e32 vcc, %[low], %[xn]\n\t"
+      "v_sub_u32_e32 %[up], %[xh1], %[h]\n\t"
+      "v_lshlrev_b32_sdwa %[tb], %[three], %[nr] dst_sel:DWORD dst_unused:UNUSED_PAD "
+      "src0_sel:DWORD src1_sel:WORD_0\n\t"
+      "v_mbcnt_lo_u32_b32 %[pos], vcc_lo, %[at]\n\t"
+      "v_mbcnt_hi_u32_b32 %[pos], vcc_hi, %[pos]\n\t"
+      "v_lshlrev_b32_e32 %[pos], 1, %[pos]"
+      : [f] "=&v"(f), [h] "=&v"(h), [t] "=&v"(t), [xn] "=&v"(u.xn), [up] "=&v"(u.up),
+        [tb] "=&v"(u.tbase), [pos] "=&v"(u.pos), [un] "=&s"(unused), "=s"(m)
+      : [lo] "v"(lo), [hi] "v"(hi), [x] "v"(x), [xh1] "v"(xh1), [pre] "v"(pre),
+        [low] "s"(kStateLow), [at] "v"(at), [three] "v"(3u), [nr] "v"(next_rec));
+  u.m = m;
+  return u;
+}
+
+// What a step computes behind its ring read: the v_perm_b32 selector of the
+// refill (bytes (x1, x0, w1, w0) in the lanes of m, the state's four
+// elsewhere), the stream position rp past the refill (the same in every lane),
+// the word that replaces the record (see dec_step; the symbol is the low half
+// of entry word hi, plus up), the escapes so far, and the lanes whose entry was
+// dense.  One asm block, since the compiler would sink most of it into the
+// next entry read's shadow, which is full; vector bit counts, since a scalar
+// one waits for the compare and its result for the next vector operation.
+struct StepShadow {
+  uint32_t sel, rp, word, esc;
+  uint64_t dense;
+};
+
+__device__ __forceinline__ StepShadow step_shadow(uint64_t m, uint32_t hi, uint32_t up,
+                                                  uint32_t rp, uint32_t rec, uint32_t esc) {
+  StepShadow r;
+  uint32_t sym;
+  register uint64_t vcc asm("vcc") = m;
+  asm("v_cndmask_b32_e32 %[sel], %[keep], %[shift], vcc\n\t"
+      "v_bcnt_u32_b32 %[rpo], vcc_lo, %[rp]\n\t"
+      "v_bcnt_u32_b32 %[rpo], vcc_hi, %[rpo]\n\t"
+      "v_add_u32_sdwa %[sym], %[up], %[hi] dst_sel:DWORD dst_unused:UNUSED_PAD "
+      "src0_sel:DWORD src1_sel:WORD_0\n\t"
+      "v_cmp_eq_u32_sdwa vcc, %[sym], %[rec] src0_sel:DWORD src1_sel:WORD_1\n\t"
+      "v_lshl_or_b32 %[word], %[esc], 16, %[sym]\n\t"
+      "v_cmp_le_u32_e64 %[dn], %[dmin], %[hi]\n\t"
+      "v_bcnt_u32_b32 %[esco], vcc_lo, %[esc]\n\t"
+      "v_bcnt_u32_b32 %[esco], vcc_hi, %[esco]"
+      : [sel] "=&v"(r.sel), [rpo] "=&v"(r.rp), [sym] "=&v"(sym), [word] "=&v"(r.word),
+        [esco] "=&v"(r.esc), [dn] "=&s"(r.dense), "+s"(vcc)
+      : [keep] "v"(0x07060504u), [shift] "v"(0x05040100u), [rp] "v"(rp), [up] "v"(up),
+        [hi] "v"(hi), [rec] "v"(rec), [esc] "v"(esc), [dmin] "s"(0xffff0000u));
+  return r;
+}
+
+// A block of SB steps in the common case (every lane active, every table in
+// LDS), bucket lookups.  rec: LDS address of the lane's first record (the
+// next steps' are 4 kLanes bytes apart; rn and r2 are the first two); the
+// decoded symbol indexes replace the records.  esc: as in dec_step.
+//
+// The steps form one chain: the entry read, the state update, the refill rank
+// and the ring read.  What the next state does not need is issued while one
+// of the two reads is in flight (each takes 52 cycles and more): the decoded
+// symbol, the escape mask, the refill count and the next step's bucket base
+// behind the ring read; the symbol's store, the record two steps ahead and the
+// dense test of the step before behind the entry read.
+// The dense lanes of a step take one of three ways (kDense):
+//  - kDenseLate (wide lookups): their state is a guess until the test, after
+//    the next step's entry read; a dense step is then looked up one level down
+//    and its update, ring read and the next entry read are redone.  The test
+//    and its branch (about 40 cycles) are off the chain, a dense step costs
+//    about 265 cycles.
+//  - kDenseTwo (wide lookups, all sub-blocks of the unit's tables in LDS):
+//    every step reads a second entry, the dense lanes' from their sub-block,
+//    the others' their own again: about 75 cycles each step, no branch.
+//  - kDenseTest (256-value buckets, two levels down): the test comes before the
+//    update.
+// Returns how many steps (kDenseLate) or lanes (kDenseTwo) were dense.
+constexpr int kDenseLate = 0, kDenseTwo = 1, kDenseTest = 2;
+
+template <int SB, int kDense, uint32_t kLutOff>
+__device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint32_t rn,
+                                              uint32_t r2, uint32_t sub_addr, uint32_t& x,
+                                              int& rp_io, uint32_t& esc) {
+  constexpr bool kWide = kDense != kDenseTest;
+  constexpr int kB = kWide ? kWideBits : kLutBits;
+  constexpr bool kLate = kDense == kDenseLate;
+  constexpr uint32_t kPos = (uint32_t)(DecGeom<SB>::kRing - 1);
+  __attribute__((address_space(3))) uint32_t* recs = lds_ptr<uint32_t>(rec);
+  auto entry_addr = [&](uint32_t tbase) {
+    // the entry's LDS address (less kLutOff): bucket base + bucket
+    uint32_t addr;
+    asm("v_bfe_u32 %0, %1, %3, %4\n\tv_lshl_add_u32 %0, %0, 3, %2"
+        : "=&v"(addr)
+        : "v"(x), "v"(tbase), "n"(16 - kB), "n"(kB));
+    return addr;
+  };
+  uint32_t rp = (uint32_t)rp_io, dense_n = 0u;
+  uint32_t tbase = (rn & 0xffffu) << 3;
+  // the step before: state, entry, record, stream position, escapes, dense
+  // lanes, and its word to store
+  uint32_t x0 = 0u, r = 0u, rp0 = 0u, esc0 = 0u, word = 0u;
+  u32x2 e0 = {0u, 0u};
+  uint64_t dense = 0ull;
+  auto redo = [&]() {
+    const uint64_t d = dense_lookup<true, kWide>(tb, ((uint64_t)e0.y << 32) | e0.x, x0 & 0xffffu,
+                                                 e0.y >= 0xffff0000u);
+    const StepUpdate n = step_update((uint32_t)d, (uint32_t)(d >> 32), x0, rp0 & kPos, 0u);
+    const uint32_t w = *lds_ptr<uint16_t>(n.pos);
+    const StepShadow h = step_shadow(n.m, (uint32_t)(d >> 32), n.up, rp0, r, esc0);
+    word = h.word;
+    rp = h.rp;
+    esc = h.esc;
+    x = __builtin_amdgcn_perm(n.xn, w, h.sel);
+    ++dense_n;
+  };
+#pragma unroll
+  for (int u = 0; u < SB; ++u) {
+    uint32_t addr = entry_addr(tbase);
+    u32x2 e = *lds_ptr<u32x2>(addr + kLutOff);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kLate && u > 0 && __builtin_expect(dense != 0ull, 0)) {
+      redo();
+      addr = entry_addr(tbase);
+      e = *lds_ptr<u32x2>(addr + kLutOff);
+      asm volatile("" : "+v"(e));  // keeps this read here and the first one above the branch
+    }
+    if (u > 0) recs[(u - 1) * kLanes] = word;
+    r = rn;
+    rn = r2;
+    if (u + 2 < SB) r2 = recs[(u + 2) * kLanes];
+    if constexpr (kDense == kDenseTwo) {
+      // sub-block e.x, sub-range (cum >> 1) & 15
+      static_assert(kWideSubShift == 1 && kSubBits == 4 && kSubBytes == 128, "sub-block address");
+      const uint32_t sub = ((x << 2) & 0x78u) + sub_addr;
+      __builtin_amdgcn_sched_barrier(0);
+      const bool dn = e.y >= 0xffff0000u;
+      dense_n += (uint32_t)__popcll(ballot(dn));
+      e = *lds_ptr<u32x2>((dn ? (e.x << 7) + sub : addr) + kLutOff);
+    }
+    if constexpr (kDense == kDenseTest) {
+      const bool dn = e.y >= 0xffff0000u;
+      if (__builtin_expect(ballot(dn) != 0ull, 0)) {
+        const uint64_t d =
+            dense_lookup<true, kWide>(tb, ((uint64_t)e.y << 32) | e.x, x & 0xffffu, dn);
+        e.x = (uint32_t)d;
+        e.y = (uint32_t)(d >> 32);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const StepUpdate n = step_update(e.x, e.y, x, rp & kPos, rn);
+    const uint32_t w = *lds_ptr<uint16_t>(n.pos);
+    __builtin_amdgcn_sched_barrier(0);
+    const StepShadow h = step_shadow(n.m, e.y, n.up, rp, r, esc);
+    if (kLate) {
+      dense = h.dense;
+      e0 = e;
+      x0 = x;
+      rp0 = rp;
+      esc0 = esc;
+    }
+    word = h.word;
+    rp = h.rp;
+    esc = h.esc;
+    tbase = n.tbase;
+    __builtin_amdgcn_sched_barrier(0);
+    x = __builtin_amdgcn_perm(n.xn, w, h.sel);  // x << 16 | w, or x
+  }
+  if (kLate && __builtin_expect(dense != 0ull, 0)) redo();
+  recs[(SB - 1) * kLanes] = word;
+  rp_io = uni((int)rp);
+  return dense_n;
 }
 
 // Waves per SIMD the decoder is built for: 6 (see the LDS plan); the
@@ -2348,7 +2546,7 @@ constexpr int kDecWavesPerSimd = 5;
 constexpr int kDecWavesPerSimd = 6;
 #endif
 
-template <int kMode, bool kImplicit, int SB, bool kSearch, bool kWide, bool kSkip = false>
+template <int kMode, bool kImplicit, int SB, bool kSearch, bool kWide>
 __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArgs a) {
   constexpr bool kLatents = kMode != kModeSymbols;  // fp32 output with a per-element add
   using G = DecGeom<SB>;
@@ -2357,14 +2555,12 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
   extern __shared__ __align__(16) uint8_t smem[];
   uint16_t* sring = reinterpret_cast<uint16_t*>(smem);
   uint32_t* sring32 = reinterpret_cast<uint32_t*>(smem);
-  uint2* recs = reinterpret_cast<uint2*>(smem + G::kRingBytes);
+  uint32_t* recs = reinterpret_cast<uint32_t*>(smem + G::kRingBytes);
   uint32_t* fifo = reinterpret_cast<uint32_t*>(smem + G::kRingBytes + G::kRecBytes);
-  uint8_t* after_fifo = smem + G::kRingBytes + G::kRecBytes + G::kEscBytes;
-  float* med = reinterpret_cast<float*>(after_fifo);
-  uint4* escm = reinterpret_cast<uint4*>(after_fifo + (kLatents ? G::kMedBytes : 0));
-  uint32_t* part = reinterpret_cast<uint32_t*>(escm + 2 * SB);
+  uint32_t* part =
+      reinterpret_cast<uint32_t*>(smem + G::kRingBytes + G::kRecBytes + G::kEscBytes);
   uint32_t* ctl = part + kDecPartBytes / 4;
-  uint8_t* tsm = smem + G::fixed(kLatents);
+  uint8_t* tsm = smem + G::kFixed;
   // [luts][meta][sub-blocks], or with the search lookups [bucket entries]
   // [meta][starts]: every part 16-byte aligned
   static_assert(!(kSearch && kWide), "the search lookups have no wide form");
@@ -2377,7 +2573,7 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
   uint64_t* lsub = reinterpret_cast<uint64_t*>(tsm + (kLutEntry * kLB + 16) * a.nt_cap);
   // the starts' LDS offset in one scalar register (the compiler would split
   // it into a register and a constant, one add more per lookup)
-  int starts_off = G::fixed(kLatents) + (kLutEntry * kLB + 16) * a.nt_cap;
+  int starts_off = G::kFixed + (kLutEntry * kLB + 16) * a.nt_cap;
   asm("" : "+s"(starts_off));
   uint16_t* lstarts = reinterpret_cast<uint16_t*>(smem + starts_off);
   float* scl = reinterpret_cast<float*>(smem + a.scales_lds);  // Gaussian: scale table
@@ -2485,9 +2681,9 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
                          ((beg & 3u) != 0u) | (cb < 4 * nst) | (((cb - 4 * nst) & 3) != 0);
   status |= (ok & bad_range) ? GAANS_ST_CORRUPT : 0u;
   ok = ok & !bad_range;
-  Stream S;  // the coder's; its final position is checked after the last barrier
-  S.rp = 0;
-  S.q = 0;
+  int rp = 0;  // the coder's stream position, checked after the last barrier
+  int q16 = 0;  // u16 words after the states (even)
+  const uint32_t* s32 = nullptr;  // the words
   // each wave's hash, status and escape nibbles -> part, before its last
   // barrier; the mappers publish before they issue the last block's stores,
   // since a wait for loads (the reductions') also waits for stores issued
@@ -2504,34 +2700,45 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
   };
   if (ok) {
     const uint8_t* cdata = a.payload + a.header_bytes + beg;
-    const uint32_t* s32 = reinterpret_cast<const uint32_t*>(cdata + 4 * nst);
+    s32 = reinterpret_cast<const uint32_t*>(cdata + 4 * nst);
     const uint32_t* safe = reinterpret_cast<const uint32_t*>(cdata);
-    const int q16 = (int)((cb - 4 * nst) / 2);  // u16 words after the states (even)
+    q16 = (int)((cb - 4 * nst) / 2);
+
+    // Per mapped step, kept by its mapper until it stores the step two blocks
+    // later (o0, f0, m0: the block to store; o1, f1, m1: the one mapped last):
+    // the table's offset, its escape symbol (s0, s1) as the coder sees it, its
+    // symbol 0's starts index (search) and the median or mean.
+    uint32_t o0[kPer], o1[kPer], s0[kPer], s1[kPer], f0[kPer], f1[kPer];
+    float m0[kPer], m1[kPer];
 
     // decoded values of block j -> HBM, escapes resolved first
     auto store_block = [&](int j, bool last) {
-      const uint2* src = recs + (j & 1) * SB * kLanes;
+      const uint32_t* src = recs + (j & 1) * SB * kLanes;
       const bool any_esc = uni((int)ctl[4 + (j & 1)]) != 0;
       const uint32_t avail = (uint32_t)uni((int)ctl[1]);
       uint32_t vals[kPer];
+      const uint32_t at = any_esc ? (uint32_t)uni((int)ctl[10 + (j & 1)]) : 0u;
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
         const int u = (wid - 1) + kMappers * e;
         if (SB % kMappers != 0 && u >= SB) break;
-        const uint2 r = src[u * kLanes + lane];
-        // the coder's value: in x, or with the search lookups in y (x keeps
-        // the table's first segment, whose table's offset the escape mapping
-        // needs)
-        uint32_t v = kSearch ? r.y : r.x;
-        if (any_esc && j * SB + u < T) {
-          const uint4 ei = escm[(j & 1) * SB + u];  // escaping lanes, first entry
-          const uint64_t em = (uint64_t)(uint32_t)uni((int)ei.x) |
-                              ((uint64_t)(uint32_t)uni((int)ei.y) << 32);
-          if (em) {
-            const uint32_t off =
-                kSearch ? tb.lmeta[(r.x & 0xffffu) / (uint32_t)kSearchEntries].z : r.y;
-            esc_resolve<R>(em, (uint32_t)uni((int)ei.z), off, v, avail, fifo, enib, status, lane);
-          }
+        const uint32_t word = src[u * kLanes + lane];  // the coder's
+        const uint32_t sym = word & 0xffffu;
+        uint32_t v = sym + o0[e] - (kSearch ? f0[e] : 0u);
+        uint64_t em = 0;
+        if (any_esc) {  // the step's escaping lanes and its first escape entry
+          em = ballot(lane + kLanes * (j * SB + u) < len && sym == s0[e]);
+          if (em)
+            esc_resolve<R>(em, at + (uint32_t)uni((int)(word >> 16)), o0[e], v, avail, fifo, enib,
+                           status, lane);
+        }
+        // an ordinary symbol's value (sym < 2^16) overflows int32 exactly when
+        // it wraps below the offset
+        if (!offsets_safe) {
+          const bool oob = lane + kLanes * (j * SB + u) < len && !((em >> lane) & 1ull) &&
+                           (int32_t)v < (int32_t)o0[e];
+          status |= oob ? GAANS_ST_CORRUPT : 0u;
+          v = oob ? 0u : v;
         }
         vals[e] = v;
       }
@@ -2544,15 +2751,14 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
         if (p < len) {
           const int64_t i = row + unit_pos(start, (int32_t)a.S, p);
           if (kLatents)
-            a.out_y[i] = __fadd_rn((float)(int32_t)vals[e],
-                                   med[((j & 1) * SB + u) * kLanes + lane]);
+            a.out_y[i] = __fadd_rn((float)(int32_t)vals[e], m0[e]);
           else a.out_sym[i] = (int32_t)vals[e];
         }
       }
     };
     GaussCoarse gc{};  // the mappers': the scale table's coarse level
     auto map_block = [&](int j) {
-      uint2* dst = recs + (j & 1) * SB * kLanes;
+      uint32_t* dst = recs + (j & 1) * SB * kLanes;
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
         const int u = (wid - 1) + kMappers * e;
@@ -2562,16 +2768,17 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
                                ? gauss_index(__int_as_float(cbx[e]), scl, a.n_scales,
                                              a.scales_pow2, a.scale_bound, gc)
                                : cbx[e];
-        uint2 r;
+        uint32_t r;
         if constexpr (kSearch) {
-          r = dec_record_search(a, tb, lane, j * SB + u, len, ix, hash, status);
+          r = dec_record_search(a, tb, lane, j * SB + u, len, ix, hash, status, o1[e], f1[e]);
           all_lds = true;
         } else {
           r = dec_record<kImplicit, kWide>(a, tb, lane, j * SB + u, len, start, ix, hash,
-                                           status, all_lds);
+                                           status, all_lds, o1[e]);
         }
         dst[u * kLanes + lane] = r;
-        if (kLatents) med[((j & 1) * SB + u) * kLanes + lane] = cm[e];
+        s1[e] = r >> 16;
+        m1[e] = cm[e];
         if (!all_lds && lane == 0)
           __hip_atomic_fetch_or(&ctl[2 + (j & 1)], 1u << u, __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -2579,23 +2786,21 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
     };
 
     // Loads that do not depend on the tables are issued before the tables are
-    // staged, so that they overlap: the coder's initial states and first
-    // stream words, the mappers' first two blocks of inputs, the escape
-    // reader's window.
+    // staged, so that they overlap: the coder's initial states, the mappers'
+    // first two blocks of inputs, the last wave's first stream words and
+    // escape window.
     EscReader E;
+    Stream S;
     uint32_t x = kStateLow;
-    uint32_t w0[G::kPre][G::kPfU32];
     if (wid == 0) {
+      x = safe[lane < A ? lane : 0];  // lanes >= A: below
+    } else if (wid == kEscWave) {
       S.s32 = s32;
       S.lane_off = 4u * (uint32_t)lane;
       S.q = q16;
       S.q32 = q16 / 2;
       S.filled = 0;
-      x = safe[lane < A ? lane : 0];  // lanes >= A: below
-#pragma unroll
-      for (int b = 0; b < G::kPre; ++b) stream_batch32<G::kPfU32>(S, b * (G::kPfWords / 2), w0[b]);
-      stream_batch32<G::kPfU32>(S, G::kPre * (G::kPfWords / 2), S.pf);
-    } else if (wid == kEscWave) {
+      stream_batch32<G::kPfU32>(S, 0, S.pf);
       E.w32 = s32;
       E.n32 = q16 / 2;
       E.base = 0;
@@ -2605,7 +2810,7 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
       E.w0 = esc_word(E, lane);
       E.w1 = esc_word(E, kLanes + lane);
     }
-    if (tid < 8) ctl[tid] = tid == 1 ? kAllAvail : 0u;
+    if (tid < kDecCtlBytes / 4) ctl[tid] = tid == 1 ? kAllAvail : 0u;
     if (kMode == kModeGaussian) stage_scales<kDecThreads>(scl, a.scale_table, a.n_scales, tid);
     stage_late<kDecThreads, kSearch>(tb, est, lmeta, a.nd_cap ? lsub : nullptr,
                                      (uint32_t)a.nd_cap, bd, tid);
@@ -2618,13 +2823,15 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
     // last store.
     if (wid == 0) {
       x = lane < A ? x : kStateLow;
-#pragma unroll
-      for (int b = 0; b < G::kPre; ++b)
-#pragma unroll
-        for (int kk = 0; kk < G::kPfU32; ++kk)
-          sring32[(b * (G::kPfWords / 2) + kk * kLanes + lane) & (G::kRing / 2 - 1)] = w0[b][kk];
-      S.filled = G::kPre * G::kPfWords;
       uint32_t ecur = 0;  // escape entries consumed
+      // Wide lookups: which way the next block's dense lanes go, by how many
+      // the last one had (a channel's table decides, and a chunk's channels
+      // differ).  kDenseTwo costs what kDenseLate does at three dense steps in
+      // ten.  sub_addr: LDS address of sub-block 0 of the blob, less kFixed.
+      const bool two_ok = kWide && bd.d1 > bd.d0 && tb.sub_n == bd.d1 - bd.d0;
+      bool two = false;
+      const uint32_t sub_addr = (uint32_t)((kLutEntry * kLB + 16) * a.nt_cap) -
+                                (uint32_t)kSubBytes * tb.sub_first;
       // The coder's chain of dependent steps bounds the block loop; its
       // instructions go first when mapper or escape waves of this or another
       // workgroup on the CU compete for the same SIMD.
@@ -2633,71 +2840,61 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
       pc.mark(3);
       pc.cycles(12);
       for (int j = 0; j < nblk; ++j) {
-        uint2* src = recs + (j & 1) * SB * kLanes;
-        uint4* ei = escm + (j & 1) * SB;
-        uint2 r[SB];
-        uint32_t ov[SB];
-#pragma unroll
-        for (int u = 0; u < SB; ++u) r[u] = src[u * kLanes + lane];
+        uint32_t* src = recs + (j & 1) * SB * kLanes;
+        const uint32_t rn = src[lane], r2 = src[kLanes + lane];
         // steps whose tables are not all in LDS; cleared for block j + 2 (the
         // search lookups stage every table: no read, no wait)
         const uint32_t nl = kSearch ? 0u : (uint32_t)uni((int)ctl[2 + (j & 1)]);
         if (!kSearch) ctl[2 + (j & 1)] = 0u;  // every lane: no exec-mask branch
-        // after the block's LDS reads: the compiler makes the first LDS read
-        // after the prefetch loads wait for them, so they are issued after
-        // the records are read and return during the block's steps
-        stream_block_start<SB>(S, sring32, lane);
-        uint64_t any_em = 0;
-        if ((j + 1) * SB * kLanes <= len && nl == 0 && offsets_safe) {
-          // common case: every lane of the block active, LDS tables, no
-          // per-step branches
-          uint64_t em[SB];
+        uint32_t esc = 0u;  // escapes of the block
+        if ((j + 1) * SB * kLanes <= len && nl == 0) {
+          // common case: every lane of the block active, LDS tables
+          if constexpr (kSearch) {
+            uint32_t r[SB], ov[SB];
 #pragma unroll
-          for (int u = 0; u < SB; ++u) {
-            ov[u] = dec_step<true, true, SB, kSearch, kWide, kSkip>(tb, r[u], x, S, sring, em[u],
-                                                                 status, lane);
-            any_em |= em[u];
-          }
-          if (__builtin_expect(any_em != 0ull, 0)) {
+            for (int u = 0; u < SB; ++u) r[u] = src[u * kLanes + lane];
 #pragma unroll
-            for (int u = 0; u < SB; ++u) {
-              if (lane == 0) ei[u] = make_uint4((uint32_t)em[u], (uint32_t)(em[u] >> 32), ecur, 0u);
-              ecur += (uint32_t)__popcll(em[u]);
+            for (int u = 0; u < SB; ++u)
+              ov[u] = dec_step<true, true, SB, true>(tb, r[u], x, rp, esc);
+#pragma unroll
+            for (int u = 0; u < SB; ++u) src[u * kLanes + lane] = ov[u];
+          } else {
+            const uint32_t rec =
+                (uint32_t)G::kRingBytes + 4u * (uint32_t)((j & 1) * SB * kLanes + lane);
+            constexpr uint32_t kLut = (uint32_t)G::kFixed;
+            if constexpr (!kWide) {
+              dec_block<SB, kDenseTest, kLut>(tb, rec, rn, r2, 0u, x, rp, esc);
+            } else if (two) {
+              two = dec_block<SB, kDenseTwo, kLut>(tb, rec, rn, r2, sub_addr, x, rp, esc) * 4u >=
+                    (uint32_t)SB;
+            } else {
+              two = dec_block<SB, kDenseLate, kLut>(tb, rec, rn, r2, 0u, x, rp, esc) * 10u >=
+                        3u * (uint32_t)SB &&
+                    two_ok;
             }
-          }
-          // decoded values replace the records' x words (y with the search
-          // lookups); the mappers store them
-#pragma unroll
-          for (int u = 0; u < SB; ++u) {
-            if constexpr (kSearch) src[u * kLanes + lane].y = ov[u];
-            else src[u * kLanes + lane].x = ov[u];
           }
         } else {
           // last block or tables outside LDS: one step at a time
 #pragma unroll 1
           for (int u = 0; u < SB && j * SB + u < T; ++u) {
-            const uint2 ru = src[u * kLanes + lane];
-            uint64_t em;
+            const uint32_t ru = src[u * kLanes + lane];
             uint32_t v;
             if constexpr (kSearch) {
-              v = dec_step<true, false, SB, true>(tb, ru, x, S, sring, em, status, lane);
+              v = dec_step<true, false, SB, true>(tb, ru, x, rp, esc);
             } else {
               v = ((nl >> u) & 1u) == 0u
-                      ? dec_step<true, false, SB, false, kWide>(tb, ru, x, S, sring, em, status,
-                                                               lane)
-                      : dec_step<false, false, SB, false, kWide>(tb, ru, x, S, sring, em, status,
-                                                                lane);
+                      ? dec_step<true, false, SB, false, kWide>(tb, ru, x, rp, esc)
+                      : dec_step<false, false, SB, false, kWide>(tb, ru, x, rp, esc);
             }
-            if (lane == 0) ei[u] = make_uint4((uint32_t)em, (uint32_t)(em >> 32), ecur, 0u);
-            ecur += (uint32_t)__popcll(em);
-            any_em |= em;
-            if constexpr (kSearch) src[u * kLanes + lane].y = v;
-            else src[u * kLanes + lane].x = v;
+            src[u * kLanes + lane] = v;
           }
         }
         // every lane writes the same (uniform) values: no exec-mask branch
-        ctl[4 + (j & 1)] = any_em != 0ull ? 1u : 0u;
+        ctl[4 + (j & 1)] = esc;
+        ctl[10 + (j & 1)] = ecur;
+        ecur += esc;
         ctl[6 + ((j + 1) & 1)] = ecur;
+        ctl[8 + ((j + 1) & 1)] = (uint32_t)rp;
         pc.bar_in();
         __syncthreads();
         pc.bar_out();
@@ -2708,13 +2905,16 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
       publish();
       __syncthreads();  // after the mappers' last store
     } else if (wid == kEscWave) {
+      if (S.q > 0) stream_commit<SB>(S, sring32, lane);  // block 0's words
       __syncthreads();
       for (int j = 0; j < nblk; ++j) {
+        stream_block<SB>(S, uni((int)ctl[8 + (j & 1)]), sring32, lane);
         // the entries of block j: at most SB kLanes past those consumed before it
         esc_parse<R>(E, (uint32_t)uni((int)ctl[6 + (j & 1)]) + (uint32_t)(SB * kLanes), fifo, ctl,
                      lane);
         __syncthreads();
       }
+      if (lane == 0) ctl[0] = (uint32_t)S.filled;
       publish();
       __syncthreads();
     } else {
@@ -2724,6 +2924,13 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
       for (int j = 0; j < nblk; ++j) {
         // mappers: store block j - 1 and map block j + 1 while the coder decodes block j
         if (j > 0) store_block(j - 1, false);
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+          o0[e] = o1[e];
+          s0[e] = s1[e];
+          f0[e] = f1[e];
+          m0[e] = m1[e];
+        }
         if (j + 1 < nblk) {
 #pragma unroll
           for (int e = 0; e < kPer; ++e) {
@@ -2758,23 +2965,24 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
       // stream, pad and escape words consumed exactly (eq escape nibbles);
       // the pad word and the unused nibbles of the last escape word are zero
       const int qe = (int)((eq + 3u) >> 2);
-      const int pad = (S.rp + qe) & 1;
-      if (S.rp + qe + pad != S.q) {
+      const int pad = (rp + qe) & 1;
+      const int filled = (int)ctl[0];
+      if (rp + qe + pad != q16) {
         st |= GAANS_ST_CORRUPT;
       } else {
         // u16 word i of the stream: from the ring while it still holds it
         // (the ring keeps the last kRing words committed, [filled - kRing,
         // filled)), else from global memory
-        const uint16_t* s16 = reinterpret_cast<const uint16_t*>(S.s32);
+        const uint16_t* s16 = reinterpret_cast<const uint16_t*>(s32);
         auto word16 = [&](int i) -> uint32_t {
-          if (i < S.filled && i >= S.filled - G::kRing) return sring[i & (G::kRing - 1)];
+          if (i < filled && i >= filled - G::kRing) return sring[i & (G::kRing - 1)];
           return s16[i];
         };
-        if (pad && word16(S.rp) != 0) st |= GAANS_ST_CORRUPT;
+        if (pad && word16(rp) != 0) st |= GAANS_ST_CORRUPT;
         if (eq & 3u) {
           // escape u32 eq >> 3 holds the first unused nibble (in range: the
           // words were consumed exactly); its halves are swapped in the stream
-          const int m = S.q32 - 1 - (int)(eq >> 3);
+          const int m = q16 / 2 - 1 - (int)(eq >> 3);
           const uint32_t v = word16(2 * m + 1) | (word16(2 * m) << 16);
           const uint32_t last = v >> (4u * (eq & 7u));
           if (last & ((1u << (4u * (4u - (eq & 3u)))) - 1u)) st |= GAANS_ST_CORRUPT;
@@ -3276,8 +3484,7 @@ int64_t search_lds(const gaans_tables* t, uint32_t* starts_words) {
   return (int64_t)t->M * (4 * kSearchEntries + 16) + sb;
 }
 
-DecPlan plan_decode(const gaans_tables* t, int64_t P, int64_t units, bool latents,
-                    const DevLds& d, int64_t extra = 0, bool range_ok = true,
+DecPlan plan_decode(const gaans_tables* t, int64_t P, int64_t units, const DevLds& d, int64_t extra = 0, bool range_ok = true,
                     bool search_ok = false) {
   const int64_t per_table = 8 * kLutSize + 16;
   const int64_t per_wide = 8 * kWideSize + 16;
@@ -3300,7 +3507,7 @@ DecPlan plan_decode(const gaans_tables* t, int64_t P, int64_t units, bool latent
     const int64_t typical = (P * t->total_wide + t->M - 1) / t->M * 3 / 2;
     for (int subs = 2; wide_ok && subs >= 0; --subs)
       for (int sb = 16; sb >= 8; sb >>= 1) {
-        const int64_t fixed = dec_fixed_lds(latents, sb);
+        const int64_t fixed = dec_fixed_lds(sb);
         Stage s;
         if (!fit_stage(t, P, per_wide, 0, subs == 2 ? kSubBytes : 0, cap - fixed - extra, &s,
                        range_ok, true))
@@ -3316,7 +3523,7 @@ DecPlan plan_decode(const gaans_tables* t, int64_t P, int64_t units, bool latent
       }
     for (int opt = 0; opt < 9; ++opt) {
       const int sb = 16 >> (opt % 3);  // 16-, 8-, then 4-step blocks of each kind
-      const int64_t fixed = dec_fixed_lds(latents, sb);
+      const int64_t fixed = dec_fixed_lds(sb);
       if (opt >= 3 && !has_dense) break;  // same as the options already tried
       if (opt >= 3 && opt < 6) {
         if (search_ok && fixed + search_bytes + extra <= cap)
@@ -3332,7 +3539,7 @@ DecPlan plan_decode(const gaans_tables* t, int64_t P, int64_t units, bool latent
                        false, 0, false};
     }
   }
-  return DecPlan{Stage{0, 0, 0, 0}, 8, (size_t)dec_fixed_lds(latents, 8), false, 0, false};
+  return DecPlan{Stage{0, 0, 0, 0}, 8, (size_t)dec_fixed_lds(8), false, 0, false};
 }
 
 // Allow dynamic LDS above the default limit (once per kernel and device).
@@ -3416,18 +3623,17 @@ EncKernel enc_kernel(int mode, bool imp, int sb, int nm) {
   }
 }
 
-template <int kMode, bool kImp, bool kSearch, bool kWide = false, bool kSkip = false>
+template <int kMode, bool kImp, bool kSearch, bool kWide = false>
 DecKernel dec_kernel_sb(int sb) {
-  return sb == 4 ? k_decode<kMode, kImp, 4, kSearch, kWide, kSkip>
-                 : (sb == 8 ? k_decode<kMode, kImp, 8, kSearch, kWide, kSkip>
-                            : k_decode<kMode, kImp, 16, kSearch, kWide, kSkip>);
+  return sb == 4 ? k_decode<kMode, kImp, 4, kSearch, kWide>
+                 : (sb == 8 ? k_decode<kMode, kImp, 8, kSearch, kWide>
+                            : k_decode<kMode, kImp, 16, kSearch, kWide>);
 }
 
 // Decode kernel of a mode, index kind, block size and lookup kind (the
 // search lookups serve explicit or computed indexes only; the wide lookups
-// are staged with 8- or 16-step blocks only).  skip: the variant whose steps
-// skip the refill read when no lane refills, for the 256-bucket lookups.
-DecKernel dec_kernel(int mode, bool imp, int sb, bool search, bool wide, bool skip) {
+// are staged with 8- or 16-step blocks only).
+DecKernel dec_kernel(int mode, bool imp, int sb, bool search, bool wide) {
   if (search) {
     switch (mode) {
       case kModeGaussian: return dec_kernel_sb<kModeGaussian, false, true>(sb);
@@ -3451,17 +3657,6 @@ DecKernel dec_kernel(int mode, bool imp, int sb, bool search, bool wide, bool sk
                              : k_decode<kModeSymbols, true, 16, false, true>)
                    : (w == 8 ? k_decode<kModeSymbols, false, 8, false, true>
                              : k_decode<kModeSymbols, false, 16, false, true>);
-    }
-  }
-  if (skip) {
-    switch (mode) {
-      case kModeGaussian: return dec_kernel_sb<kModeGaussian, false, false, false, true>(sb);
-      case kModeLatents:
-        return imp ? dec_kernel_sb<kModeLatents, true, false, false, true>(sb)
-                   : dec_kernel_sb<kModeLatents, false, false, false, true>(sb);
-      default:
-        return imp ? dec_kernel_sb<kModeSymbols, true, false, false, true>(sb)
-                   : dec_kernel_sb<kModeSymbols, false, false, false, true>(sb);
     }
   }
   switch (mode) {
@@ -3681,11 +3876,10 @@ int decode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
   if ((rc = device_lds(&dl))) return rc;
   const bool gauss = mode == kModeGaussian;
   if (gauss) implicit = false;
-  const bool latents = mode != kModeSymbols;
   const int64_t extra =
       gauss ? align_up(4 * ((int64_t)n_scales + kGaussPad), 16) + 16 : 0;  // as for the encoder
   const bool search_ok = (tables->flags & GAANS_TABLES_SEARCH) != 0 && !implicit;
-  const DecPlan plan = plan_decode(tables, L.P, L.U, latents, dl, extra, !gauss, search_ok);
+  const DecPlan plan = plan_decode(tables, L.P, L.U, dl, extra, !gauss, search_ok);
   const Stage& st = plan.st;
   const size_t lds = plan.lds + (size_t)extra;
   if (lds > (size_t)dl.per_block)
@@ -3716,9 +3910,7 @@ int decode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
   a.nd_cap = st.nd_cap;
   a.stage_all = st.stage_all;
   a.starts_words = plan.starts_words;
-  // the refill-skipping steps when the grid needs more than one workgroup
-  // per CU (issue slots, not one unit's step latency, bound the launch)
-  e->kernel = dec_kernel(mode, implicit, plan.sb, plan.search, plan.wide, L.U > (int64_t)dl.cus);
+  e->kernel = dec_kernel(mode, implicit, plan.sb, plan.search, plan.wide);
   e->grid = (uint32_t)L.U;
   e->block = (uint32_t)kDecThreads;
   e->lds = lds;
