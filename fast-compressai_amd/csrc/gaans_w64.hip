@@ -19,10 +19,11 @@
 //    indexes / latents from HBM (a block ahead again, so the loads are in
 //    flight while the previous block is mapped), look the tables up, split
 //    escapes, hash the indexes and write one op record per lane and step
-//    into LDS (16 bytes for encode, 8 for decode); the decoder's mappers also
+//    into LDS (16 bytes for encode, 4 for decode); the decoder's mappers also
 //    store the decoded values a block behind.
-//  - The decoder's escape reader parses the chunk's escape section ahead of
-//    the coder into an LDS FIFO, so an escape costs the coder one LDS read.
+//  - The decoder's last wave keeps the coder's word ring filled and parses the
+//    chunk's escape section into an LDS FIFO, from which the mappers resolve the
+//    escapes when they store.
 //  - The CDF tables of the chunk's channels (or all tables, when they are
 //    few) are staged in LDS by the whole workgroup; others are read through
 //    L1/L2.
@@ -1856,13 +1857,13 @@ __device__ __forceinline__ uint32_t dec_record(const DecArgs& a, const Tabs& tb,
 
 // Mapper record with the search lookups (all tables in LDS): the table's first
 // segment (table * kSearchEntries, below 2^16 when the blob has the search
-// lookups) | starts index of its escape symbol << 16 (kNoSym past the chunk
-// end).  The coder's symbol is a starts index: offset is the table's less the
-// starts index of its symbol 0 (first).
+// lookups) | start of its escape symbol << 16 (the table's last: cum at or past
+// it decodes an escape).  The coder's symbol is a starts index: syms holds
+// symbol 0's | the escape symbol's << 16.
 __device__ __forceinline__ uint32_t dec_record_search(const DecArgs& a, const Tabs& tb, int lane,
                                                       int t, int len, int32_t in_b,
                                                       uint32_t& hash, uint32_t& status,
-                                                      uint32_t& offset, uint32_t& first) {
+                                                      uint32_t& offset, uint32_t& syms) {
   const int p = lane + kLanes * t;
   const bool act = p < len;
   int32_t tbi = in_b;
@@ -1872,9 +1873,11 @@ __device__ __forceinline__ uint32_t dec_record_search(const DecArgs& a, const Ta
   tbi = ok ? tbi : 0;
   hash += ok ? index_term((uint32_t)p, (uint32_t)tbi) : 0u;
   const uint4 lm = tb.lmeta[tbi];
-  first = lm.x + (uint32_t)(kStartsTablePad * tbi);  // starts index of symbol 0
+  const uint32_t first = lm.x + (uint32_t)(kStartsTablePad * tbi);  // starts index of symbol 0
+  const uint32_t es = first + lm.y - 1u;                            // of the escape symbol
   offset = lm.z;
-  return (uint32_t)tbi * (uint32_t)kSearchEntries | ((act ? first + lm.y - 1u : kNoSym) << 16);
+  syms = first | (es << 16);
+  return (uint32_t)tbi * (uint32_t)kSearchEntries | (((uint32_t)tb.lstarts[es] + 1u) << 16);
 }
 
 // One level down from a dense lookup entry e: entry i of its sub-block (LDS
@@ -1910,12 +1913,9 @@ __device__ __forceinline__ void lut_pick(uint64_t e, uint32_t cum, uint32_t& s, 
   fr = up ? (hi >> 16) + 1u : st1 - st0;
 }
 
-// cum -> (symbol, start, freq) in table t: the table's lookup entry of
-// bucket cum >> 8, for a dense bucket the entry of sub-range (cum >> 4) & 15
-// of its sub-block, for a dense sub-range the exact entry of value cum & 15
-// (see the blob layout).  kWide: the wide lookups, bucket cum >> 5 and, for
-// a dense bucket, sub-range (cum >> 1) & 15 of its sub-block.  t is the
-// staged table's first bucket (kLds) or the global table index.
+// The dense lanes' entries one level down (256-value buckets: sub-range (cum >>
+// 4) & 15 of the bucket's sub-block, then for a dense sub-range the exact entry
+// of value cum & 15; wide lookups: sub-range (cum >> 1) & 15, never dense).
 template <bool kLds, bool kWide>
 __device__ __forceinline__ uint64_t dense_lookup(const Tabs& tb, uint64_t e, uint32_t cum,
                                                  bool dense) {
@@ -1931,6 +1931,10 @@ __device__ __forceinline__ uint64_t dense_lookup(const Tabs& tb, uint64_t e, uin
   return e;
 }
 
+// cum -> (symbol, start, freq) in table t: the table's lookup entry of bucket
+// cum >> 8 (kWide: cum >> 5), a dense one's from its sub-block (see the blob
+// layout).  t is the staged table's first bucket (kLds) or the global table
+// index.
 template <bool kLds, bool kWide = false>
 __device__ __forceinline__ void dec_lookup(const Tabs& tb, uint32_t t, uint32_t cum, bool act,
                                            uint32_t& s, uint32_t& st, uint32_t& fr) {
@@ -2191,9 +2195,10 @@ __device__ __forceinline__ void dec_refill(bool need, uint32_t& x, int& rp) {
 // n32 - 1 - m with its halves swapped.  An entry is a count n then n nibbles
 // of raw, and n is the minimal count of raw (raw ? msb(raw) / 4 + 1 : 0).
 //
-// The coder only marks escapes: per step, the escaping lanes and the ordinal
-// of the step's first entry.  The mapper that stores the block (during the
-// next block) resolves the values from an LDS FIFO of kEscR = 2 SB kLanes
+// The coder only counts escapes: a step's words carry how many entries the
+// block's steps before it took (the ordinal of its first entry), and a lane
+// whose symbol is its table's escape bin escapes.  The mapper that stores the
+// block (during the next block) resolves the values from an LDS FIFO of kEscR = 2 SB kLanes
 // raw values (entry e in slot e mod kEscR), which the escape reader (the
 // workgroup's last wave) fills in order: during block j it parses up to
 // c_j + SB kLanes entries, c_j being the entries consumed before block j
@@ -2308,15 +2313,14 @@ __device__ __forceinline__ void esc_resolve(uint64_t em, uint32_t base, uint32_t
   enib += e ? (raw ? ((31u - (uint32_t)__clz((int)raw)) >> 2) + 2u : 1u) : 0u;
 }
 
-// One decode step of the coder wave; returns the word that replaces the record:
-// the decoded symbol index | the block's escapes before this step << 16 (esc,
-// the same in every lane, which counts this step's in; their values are
-// resolved by the mappers, off the state chain).  kFull: every lane is active.
-template <bool kLds, bool kFull, int SB, bool kSearch = false, bool kWide = false>
-__device__ __forceinline__ uint32_t dec_step(const Tabs& tb, const uint32_t r, uint32_t& x,
-                                             int& rp, uint32_t& esc) {
-  const uint32_t es = r >> 16;
-  const bool act = kFull || es != kNoSym;
+// One decode step of the coder wave, bucket or search lookups; returns the word
+// that replaces the record: the decoded symbol index | the block's escapes
+// before this step << 16 (esc, the same in every lane, which counts this
+// step's in; their values are resolved by the mappers, off the state chain).
+// act: the lane's position is inside the unit.
+template <bool kLds, int SB, bool kSearch = false, bool kWide = false>
+__device__ __forceinline__ uint32_t dec_step(const Tabs& tb, const uint32_t r, bool act,
+                                             uint32_t& x, int& rp, uint32_t& esc) {
   const uint32_t cum = x & 0xffffu;
   uint32_t s, st, fr;
   if constexpr (kSearch) dec_lookup_search(tb, r & 0xffffu, cum, act, s, st, fr);
@@ -2324,8 +2328,9 @@ __device__ __forceinline__ uint32_t dec_step(const Tabs& tb, const uint32_t r, u
   const uint32_t xn = __umul24(fr, x >> 16) + cum - st;
   x = act ? xn : x;
   dec_refill<SB>(act & (x < kStateLow), x, rp);
+  const bool e = kSearch ? cum >= r >> 16 : s == r >> 16;
   const uint32_t word = s | (esc << 16);
-  esc += (uint32_t)__popcll(ballot(act & (s == es)));
+  esc += (uint32_t)__popcll(ballot(act & e));
   return word;
 }
 
@@ -2425,9 +2430,13 @@ __device__ __forceinline__ StepShadow step_shadow(uint64_t m, uint32_t hi, uint3
 // The steps form one chain: the entry read, the state update, the refill rank
 // and the ring read.  What the next state does not need is issued while one
 // of the two reads is in flight (each takes 52 cycles and more): the decoded
-// symbol, the escape mask, the refill count and the next step's bucket base
-// behind the ring read; the symbol's store, the record two steps ahead and the
-// dense test of the step before behind the entry read.
+// symbol, the escape and refill counts behind the ring read; the symbol's store,
+// the record two steps ahead and the dense test of the step before behind the
+// entry read.  Cycles per step on MI355X with one workgroup per CU (uniform
+// 255-symbol tables, no dense steps): 335 with the compiler's step and the
+// stream, escape masks and stores on this wave, 235 so.  512x768, P = 4: 23.1
+// -> 19.7 us; 2160x3840, P = 8: 224 -> 178 us.
+//
 // The dense lanes of a step take one of three ways (kDense):
 //  - kDenseLate (wide lookups): their state is a guess until the test, after
 //    the next step's entry read; a dense step is then looked up one level down
@@ -2534,6 +2543,168 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
   recs[(SB - 1) * kLanes] = word;
   rp_io = uni((int)rp);
   return dense_n;
+}
+
+// dec_block with the search lookups (every table in LDS; see
+// dec_lookup_search).  The symbol and its range come from the six starts in
+// three aligned words that hold starts g .. g + 4 (gb = g & ~1; start 6 is
+// masked to 0xffff for even g, since it could be the next table's): with c =
+// cum - 1 and d_i = c - (start_i - 1) mod 2^16 for each,
+//   cum - start = min d_i,  next start - cum = 2^16 - max d_i
+// over any starts of the table that include the symbol's and the next one's (a
+// start above cum wraps to more than any at or below it, and the 0xffff of a
+// first symbol or the padding, start 0 or 2^16, gives d = cum, between the
+// two).  So freq - 1 = min - max - 1 mod 2^16, and x' = (freq - 1) xh + xh +
+// min: packed 16-bit differences, minima and maxima, no compare and no select.
+// The symbol's index (the count of starts past g at or below cum) is not on
+// the chain: it is computed behind the next step's reads.
+// Cycles per step on MI355X, hyperprior y (64 Gaussian tables, 12 units): 560
+// with the compiler's 71 instructions and selects and 8-step blocks, 421 so (4
+// address operations, 5 from the entry to the starts' address, 19 from the
+// starts to the ring read, three LDS round trips; 16-step blocks fit beside
+// the tables since the records are 4 bytes).  P = 16: 94.7 -> 76.9 us, P = 4:
+// 29.9 -> 26.2 us.
+template <int SB, uint32_t kLutOff>
+__device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, uint32_t rn,
+                                                 uint32_t r2, int starts_off, uint32_t& x,
+                                                 int& rp_io, uint32_t& esc) {
+  static_assert(kSearchFine == 4 && kSearchFineBits == 5 && kSearchParts == 64,
+                "segment arithmetic below");
+  constexpr uint32_t kPos = (uint32_t)(DecGeom<SB>::kRing - 1);
+  __attribute__((address_space(3))) uint32_t* recs = lds_ptr<uint32_t>(rec);
+  uint32_t rp = (uint32_t)rp_io, r = rn;
+  uint32_t tbase = (rn & 0xffffu) << 2;
+  // the step before: max(cum - (start - 1), 0) of its six starts, position g,
+  // the mask of its word 2 and the escapes before it
+  uint32_t v0 = 0u, v1 = 0u, v2 = 0u, g0 = 0u, even0 = 0u, esc0 = 0u;
+  // its symbol (a starts index: g plus the starts past g at or below cum --
+  // even g: v0's high half, v1 and v2's low; odd: v1 and v2) | escapes << 16
+  auto word0 = [&]() {
+    uint32_t t, w;
+    asm("v_pk_min_u16 %[v0], %[v0], %[one]\n\t"
+        "v_pk_min_u16 %[v1], %[v1], %[one]\n\t"
+        "v_pk_min_u16 %[v2], %[v2], %[one]\n\t"
+        "v_and_b32_e32 %[v0], %[even], %[v0]\n\t"
+        "v_pk_add_u16 %[t], %[v1], %[v2]\n\t"
+        "v_pk_add_u16 %[t], %[t], %[v0]\n\t"
+        "v_add_u32_sdwa %[w], %[g], %[t] dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:DWORD src1_sel:WORD_0\n\t"
+        "v_add_u32_sdwa %[w], %[w], %[t] dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:DWORD src1_sel:WORD_1\n\t"
+        "v_lshl_or_b32 %[w], %[esc], 16, %[w]"
+        : [v0] "+v"(v0), [v1] "+v"(v1), [v2] "+v"(v2), [t] "=&v"(t), [w] "=&v"(w)
+        : [one] "s"(0x00010001u), [even] "v"(even0), [g] "v"(g0), [esc] "v"(esc0));
+    return w;
+  };
+#pragma unroll
+  for (int u = 0; u < SB; ++u) {
+    // entries of cum's 256-value bucket and of its 32-value part
+    uint32_t ab, ap;
+    asm("v_bfe_u32 %0, %2, 8, 8\n\tv_lshl_add_u32 %0, %0, 2, %3\n\t"
+        "v_bfe_u32 %1, %2, 5, 6\n\tv_lshl_add_u32 %1, %1, 2, %3"
+        : "=&v"(ab), "=&v"(ap)
+        : "v"(x), "v"(tbase));
+    const uint32_t eb = *lds_ptr<uint32_t>(ab + kLutOff + 4u * kSearchParts);
+    const uint32_t ep = *lds_ptr<uint32_t>(ap + kLutOff);
+    __builtin_amdgcn_sched_barrier(0);
+    r = rn;
+    rn = r2;
+    if (u + 2 < SB) r2 = recs[(u + 2) * kLanes];
+    const uint32_t cum = x & 0xffffu, xh = x >> 16, c = x - 1u;
+    const uint64_t fine = ballot((uint16_t)(cum + 1024u) < 2048u);  // cum < 1024 or >= 64512
+    if (u > 0) recs[(u - 1) * kLanes] = word0();
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t e, g, a;  // e: m | n << 8 | G << 16; g = G + ((cum & 255) m >> 8)
+    asm("v_cndmask_b32_e64 %0, %3, %4, %5\n\t"
+        "v_mul_u32_u24_sdwa %1, %6, %0 dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:BYTE_0 src1_sel:BYTE_0\n\t"
+        "v_add_u32_sdwa %1, %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:WORD_1 src1_sel:BYTE_1\n\t"
+        "v_and_b32_e32 %2, -2, %1\n\t"
+        "v_lshl_add_u32 %2, %2, 1, %7"
+        : "=&v"(e), "=&v"(g), "=&v"(a)
+        : "v"(eb), "v"(ep), "s"(fine), "v"(x), "s"(starts_off));
+    uint32_t w0 = lds_ptr<uint32_t>(a)[0], w1 = lds_ptr<uint32_t>(a)[1],
+             w2 = lds_ptr<uint32_t>(a)[2];
+    __builtin_amdgcn_sched_barrier(0);
+    // a segment no line fits: its n > 3 symbols after G are narrowed by the
+    // probes q, 2q, 3q (q = (n + 1) / 4 >= 1), four ranges a round
+    bool wide = (e & 0xffffu) > 0x3ffu;
+    if (__builtin_expect(ballot(wide) != 0ull, 0)) {
+      uint32_t nl = (e >> 8) & 0xffu;
+      do {
+        if (wide) {
+          const uint32_t q = (nl + 1u) >> 2;
+          const bool l1 = tb.lstarts[g + q] < cum, l2 = tb.lstarts[g + 2u * q] < cum,
+                     l3 = tb.lstarts[g + 3u * q] < cum;
+          const uint32_t kk = (uint32_t)l1 + (uint32_t)l2 + (uint32_t)l3;
+          g += kk * q;
+          nl = l3 ? nl - 3u * q : q - 1u;
+        }
+        wide = wide & (nl > 3u);
+      } while (ballot(wide) != 0ull);
+      a = ((g & ~1u) << 1) + (uint32_t)starts_off;
+      w0 = lds_ptr<uint32_t>(a)[0];
+      w1 = lds_ptr<uint32_t>(a)[1];
+      w2 = lds_ptr<uint32_t>(a)[2];
+      asm volatile("" : "+v"(w0), "+v"(w1), "+v"(w2));  // as for dec_block's entry
+    }
+    const uint32_t even = ((g & 1u) - 1u) << 16;  // 0xffff0000 for even g, else 0
+    const uint32_t at = rp & kPos;
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t d0, d1, d2, t, xn, pos;
+    register uint64_t m asm("vcc");
+    asm("v_or_b32_e32 %[w2], %[w2], %[even]\n\t"
+        "v_pk_sub_u16 %[d0], %[c], %[w0] op_sel_hi:[0,1]\n\t"
+        "v_pk_sub_u16 %[d1], %[c], %[w1] op_sel_hi:[0,1]\n\t"
+        "v_pk_sub_u16 %[d2], %[c], %[w2] op_sel_hi:[0,1]\n\t"
+        "v_pk_min_u16 %[t], %[d0], %[d1]\n\t"
+        "v_pk_max_u16 %[d0], %[d0], %[d1]\n\t"
+        "v_pk_min_u16 %[t], %[t], %[d2]\n\t"
+        "v_pk_max_u16 %[d0], %[d0], %[d2]\n\t"
+        "v_min_u32_sdwa %[t], %[t], %[t] dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_max_u32_sdwa %[d0], %[d0], %[d0] dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_u32_e32 %[d1], %[xh], %[t]\n\t"
+        "v_xad_u32 %[d0], %[d0], -1, %[t]\n\t"
+        "v_mad_u32_u16 %[xn], %[d0], %[xh], %[d1]\n\t"
+        "v_cmp_gt_u32_e32 vcc, %[low], %[xn]\n\t"
+        "v_lshlrev_b32_sdwa %[tb], %[two], %[rn] dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:DWORD src1_sel:WORD_0\n\t"
+        "s_nop 0\n\t"
+        "v_mbcnt_lo_u32_b32 %[pos], vcc_lo, %[at]\n\t"
+        "v_mbcnt_hi_u32_b32 %[pos], vcc_hi, %[pos]\n\t"
+        "v_lshlrev_b32_e32 %[pos], 1, %[pos]"
+        : [w2] "+v"(w2), [d0] "=&v"(d0), [d1] "=&v"(d1), [d2] "=&v"(d2), [t] "=&v"(t),
+          [xn] "=&v"(xn), [tb] "=&v"(tbase), [pos] "=&v"(pos), "=s"(m)
+        : [w0] "v"(w0), [w1] "v"(w1), [even] "v"(even), [c] "v"(c), [xh] "v"(xh),
+          [low] "s"(kStateLow), [two] "v"(2u), [rn] "v"(rn), [at] "v"(at));
+    const uint32_t w = *lds_ptr<uint16_t>(pos);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t sel, esc1;
+    asm("v_cndmask_b32_e32 %[sel], %[keep], %[shift], vcc\n\t"
+        "v_bcnt_u32_b32 %[rp], vcc_lo, %[rp]\n\t"
+        "v_bcnt_u32_b32 %[rp], vcc_hi, %[rp]\n\t"
+        "v_cmp_ge_u32_sdwa vcc, %[x], %[r] src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_pk_sub_u16 %[v0], %[x], %[w0] op_sel_hi:[0,1] clamp\n\t"
+        "v_pk_sub_u16 %[v1], %[x], %[w1] op_sel_hi:[0,1] clamp\n\t"
+        "v_pk_sub_u16 %[v2], %[x], %[w2] op_sel_hi:[0,1] clamp\n\t"
+        "v_bcnt_u32_b32 %[esc], vcc_lo, %[esci]\n\t"
+        "v_bcnt_u32_b32 %[esc], vcc_hi, %[esc]"
+        : [sel] "=&v"(sel), [rp] "+v"(rp), [esc] "=&v"(esc1), [v0] "=&v"(v0), [v1] "=&v"(v1),
+          [v2] "=&v"(v2), "+s"(m)
+        : [keep] "v"(0x07060504u), [shift] "v"(0x05040100u), [x] "v"(x), [r] "v"(r),
+          [esci] "v"(esc), [w0] "v"(w0), [w1] "v"(w1), [w2] "v"(w2));
+    g0 = g;
+    even0 = even;
+    esc0 = esc;
+    esc = esc1;
+    __builtin_amdgcn_sched_barrier(0);
+    x = __builtin_amdgcn_perm(xn, w, sel);  // x << 16 | w, or x
+  }
+  recs[(SB - 1) * kLanes] = word0();
+  rp_io = uni((int)rp);
 }
 
 // Waves per SIMD the decoder is built for: 6 (see the LDS plan); the
@@ -2706,9 +2877,9 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
 
     // Per mapped step, kept by its mapper until it stores the step two blocks
     // later (o0, f0, m0: the block to store; o1, f1, m1: the one mapped last):
-    // the table's offset, its escape symbol (s0, s1) as the coder sees it, its
-    // symbol 0's starts index (search) and the median or mean.
-    uint32_t o0[kPer], o1[kPer], s0[kPer], s1[kPer], f0[kPer], f1[kPer];
+    // the table's offset, its symbol 0 and escape symbol << 16 as the coder has
+    // them (s0, s1), and the median or mean.
+    uint32_t o0[kPer], o1[kPer], s0[kPer], s1[kPer];
     float m0[kPer], m1[kPer];
 
     // decoded values of block j -> HBM, escapes resolved first
@@ -2724,10 +2895,10 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
         if (SB % kMappers != 0 && u >= SB) break;
         const uint32_t word = src[u * kLanes + lane];  // the coder's
         const uint32_t sym = word & 0xffffu;
-        uint32_t v = sym + o0[e] - (kSearch ? f0[e] : 0u);
+        uint32_t v = sym + o0[e] - (kSearch ? s0[e] & 0xffffu : 0u);
         uint64_t em = 0;
         if (any_esc) {  // the step's escaping lanes and its first escape entry
-          em = ballot(lane + kLanes * (j * SB + u) < len && sym == s0[e]);
+          em = ballot(lane + kLanes * (j * SB + u) < len && sym == s0[e] >> 16);
           if (em)
             esc_resolve<R>(em, at + (uint32_t)uni((int)(word >> 16)), o0[e], v, avail, fifo, enib,
                            status, lane);
@@ -2770,14 +2941,14 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
                                : cbx[e];
         uint32_t r;
         if constexpr (kSearch) {
-          r = dec_record_search(a, tb, lane, j * SB + u, len, ix, hash, status, o1[e], f1[e]);
+          r = dec_record_search(a, tb, lane, j * SB + u, len, ix, hash, status, o1[e], s1[e]);
           all_lds = true;
         } else {
           r = dec_record<kImplicit, kWide>(a, tb, lane, j * SB + u, len, start, ix, hash,
                                            status, all_lds, o1[e]);
+          s1[e] = r & 0xffff0000u;
         }
         dst[u * kLanes + lane] = r;
-        s1[e] = r >> 16;
         m1[e] = cm[e];
         if (!all_lds && lane == 0)
           __hip_atomic_fetch_or(&ctl[2 + (j & 1)], 1u << u, __ATOMIC_RELAXED,
@@ -2850,14 +3021,9 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
         if ((j + 1) * SB * kLanes <= len && nl == 0) {
           // common case: every lane of the block active, LDS tables
           if constexpr (kSearch) {
-            uint32_t r[SB], ov[SB];
-#pragma unroll
-            for (int u = 0; u < SB; ++u) r[u] = src[u * kLanes + lane];
-#pragma unroll
-            for (int u = 0; u < SB; ++u)
-              ov[u] = dec_step<true, true, SB, true>(tb, r[u], x, rp, esc);
-#pragma unroll
-            for (int u = 0; u < SB; ++u) src[u * kLanes + lane] = ov[u];
+            dec_block_search<SB, (uint32_t)G::kFixed>(
+                tb, (uint32_t)G::kRingBytes + 4u * (uint32_t)((j & 1) * SB * kLanes + lane), rn,
+                r2, starts_off, x, rp, esc);
           } else {
             const uint32_t rec =
                 (uint32_t)G::kRingBytes + 4u * (uint32_t)((j & 1) * SB * kLanes + lane);
@@ -2878,13 +3044,14 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
 #pragma unroll 1
           for (int u = 0; u < SB && j * SB + u < T; ++u) {
             const uint32_t ru = src[u * kLanes + lane];
+            const bool act = lane + kLanes * (j * SB + u) < len;
             uint32_t v;
             if constexpr (kSearch) {
-              v = dec_step<true, false, SB, true>(tb, ru, x, rp, esc);
+              v = dec_step<true, SB, true>(tb, ru, act, x, rp, esc);
             } else {
               v = ((nl >> u) & 1u) == 0u
-                      ? dec_step<true, false, SB, false, kWide>(tb, ru, x, rp, esc)
-                      : dec_step<false, false, SB, false, kWide>(tb, ru, x, rp, esc);
+                      ? dec_step<true, SB, false, kWide>(tb, ru, act, x, rp, esc)
+                      : dec_step<false, SB, false, kWide>(tb, ru, act, x, rp, esc);
             }
             src[u * kLanes + lane] = v;
           }
@@ -2928,7 +3095,6 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
         for (int e = 0; e < kPer; ++e) {
           o0[e] = o1[e];
           s0[e] = s1[e];
-          f0[e] = f1[e];
           m0[e] = m1[e];
         }
         if (j + 1 < nblk) {
