@@ -1754,7 +1754,7 @@ constexpr int kDecCtlBytes = 48;
 constexpr uint32_t kNoSym = 0xffffu;  // record of a lane past the chunk end
 // words after the stream ring that repeat its first ones: a step reads at most
 // kLanes words from a position below kRing, so its reads need no wrap
-constexpr int kRingMirror = 2 * kLanes;
+constexpr int kRingMirror = kLanes;
 constexpr uint32_t kAllAvail = 0xffffffffu;
 
 struct DecArgs {
@@ -1787,7 +1787,8 @@ struct DecArgs {
 // and the steps between two barriers).
 template <int SB>
 struct DecGeom {
-  static constexpr int kPer = (SB + kMappers - 1) / kMappers;  // steps per mapper wave and block
+  static constexpr int kPer = SB / kMappers;  // steps per mapper wave and block
+  static_assert(SB % kMappers == 0, "whole steps per mapper");
   static constexpr int kBlockWords = SB * kLanes;      // a block's most words: one per lane and step
   static constexpr int kPfU32 = kBlockWords / 2 / kLanes;  // stream batch: u32 per lane
   static constexpr int kPfWords = kBlockWords;             // words per batch
@@ -1807,7 +1808,6 @@ struct DecGeom {
   // overwrites a word that block j may read.
   static_assert(kLowWater + kPfWords <= kRing && kPfU32 <= kPfU32Max,
                 "decoder stream ring too small");
-  static_assert(kRingMirror == 2 * kLanes, "a batch's first u32 per lane is the mirror");
   static_assert((kDecPartBytes + kDecCtlBytes) % 16 == 0 && kRingBytes % 16 == 0,
                 "LDS parts 16-byte aligned");
 };
@@ -1816,22 +1816,20 @@ int dec_fixed_lds(int sb) {
   return sb >= 16 ? DecGeom<16>::kFixed : (sb >= 8 ? DecGeom<8>::kFixed : DecGeom<4>::kFixed);
 }
 
-// Mapper record of one lane and step (4 bytes), tables in LDS when the step's
+// Mapper record of one lane and step (table tbi; 4 bytes), tables in LDS when the step's
 // flag is 1: the lane's table | escape symbol << 16 (nsym - 1; kNoSym for a
 // lane past the chunk end); the table is the LDS-local index times the
 // lookup's bucket count (its first bucket: one add fewer per step for the
 // coder), or the global index.  offset (the table's) stays with the mapper,
 // which stores the same lane and step later.  The coder overwrites the record
 // with the decoded symbol index.
-template <bool kImplicit, bool kWide>
+template <bool kWide>
 __device__ __forceinline__ uint32_t dec_record(const DecArgs& a, const Tabs& tb, int lane, int t,
-                                               int len, int32_t start, int32_t in_b,
-                                               uint32_t& hash, uint32_t& status, bool& all_lds,
+                                               int len, int32_t tbi, uint32_t& hash,
+                                               uint32_t& status, bool& all_lds,
                                                uint32_t& offset) {
   const int p = lane + kLanes * t;
   const bool act = p < len;
-  int32_t tbi =
-      kImplicit ? (int32_t)udiv((uint32_t)unit_pos(start, (int32_t)a.S, p), a.div_hw) : in_b;
   const bool bad = act & ((uint32_t)tbi >= a.M);
   const bool ok = act & !bad;
   status |= bad ? GAANS_ST_INDEX : 0u;
@@ -1860,24 +1858,28 @@ __device__ __forceinline__ uint32_t dec_record(const DecArgs& a, const Tabs& tb,
 // lookups) | start of its escape symbol << 16 (the table's last: cum at or past
 // it decodes an escape).  The coder's symbol is a starts index: syms holds
 // symbol 0's | the escape symbol's << 16.
+__device__ __forceinline__ uint32_t search_record(const Tabs& tb, int32_t tbi, uint32_t base,
+                                                  uint32_t nsym, uint32_t& syms) {
+  const uint32_t first = base + (uint32_t)(kStartsTablePad * tbi);
+  const uint32_t es = first + nsym - 1u;
+  syms = first | (es << 16);
+  return (uint32_t)tbi * (uint32_t)kSearchEntries | (((uint32_t)tb.lstarts[es] + 1u) << 16);
+}
+
 __device__ __forceinline__ uint32_t dec_record_search(const DecArgs& a, const Tabs& tb, int lane,
-                                                      int t, int len, int32_t in_b,
+                                                      int t, int len, int32_t tbi,
                                                       uint32_t& hash, uint32_t& status,
                                                       uint32_t& offset, uint32_t& syms) {
   const int p = lane + kLanes * t;
   const bool act = p < len;
-  int32_t tbi = in_b;
   const bool bad = act & ((uint32_t)tbi >= a.M);
   const bool ok = act & !bad;
   status |= bad ? GAANS_ST_INDEX : 0u;
   tbi = ok ? tbi : 0;
   hash += ok ? index_term((uint32_t)p, (uint32_t)tbi) : 0u;
   const uint4 lm = tb.lmeta[tbi];
-  const uint32_t first = lm.x + (uint32_t)(kStartsTablePad * tbi);  // starts index of symbol 0
-  const uint32_t es = first + lm.y - 1u;                            // of the escape symbol
   offset = lm.z;
-  syms = first | (es << 16);
-  return (uint32_t)tbi * (uint32_t)kSearchEntries | (((uint32_t)tb.lstarts[es] + 1u) << 16);
+  return search_record(tb, tbi, lm.x, lm.y, syms);
 }
 
 // One level down from a dense lookup entry e: entry i of its sub-block (LDS
@@ -2162,7 +2164,7 @@ __device__ __forceinline__ void stream_commit(Stream& S, uint32_t* ring32, int l
 #pragma unroll
   for (int kk = 0; kk < G::kPfU32; ++kk) dst[kk * kLanes] = S.pf[kk];
   // the mirror (of a batch at the ring's start; else its words once more)
-  ring32[(at ? at : (uint32_t)(G::kRing / 2)) + lane] = S.pf[0];
+  if (lane < kRingMirror / 2) ring32[(at ? at : (uint32_t)(G::kRing / 2)) + lane] = S.pf[0];
   S.filled = uni(S.filled + G::kPfWords);
   stream_batch32<G::kPfU32>(S, S.filled >> 1, S.pf);
 }
@@ -2422,7 +2424,7 @@ __device__ __forceinline__ StepShadow step_shadow(uint64_t m, uint32_t hi, uint3
   return r;
 }
 
-// A block of SB steps in the common case (every lane active, every table in
+// NS steps of a block in the common case (every lane active, every table in
 // LDS), bucket lookups.  rec: LDS address of the lane's first record (the
 // next steps' are 4 kLanes bytes apart; rn and r2 are the first two); the
 // decoded symbol indexes replace the records.  esc: as in dec_step.
@@ -2437,27 +2439,22 @@ __device__ __forceinline__ StepShadow step_shadow(uint64_t m, uint32_t hi, uint3
 // stream, escape masks and stores on this wave, 235 so.  512x768, P = 4: 23.1
 // -> 19.7 us; 2160x3840, P = 8: 224 -> 178 us.
 //
-// The dense lanes of a step take one of three ways (kDense):
-//  - kDenseLate (wide lookups): their state is a guess until the test, after
-//    the next step's entry read; a dense step is then looked up one level down
-//    and its update, ring read and the next entry read are redone.  The test
-//    and its branch (about 40 cycles) are off the chain, a dense step costs
-//    about 265 cycles.
-//  - kDenseTwo (wide lookups, all sub-blocks of the unit's tables in LDS):
-//    every step reads a second entry, the dense lanes' from their sub-block,
-//    the others' their own again: about 75 cycles each step, no branch.
-//  - kDenseTest (256-value buckets, two levels down): the test comes before the
-//    update.
-// Returns how many steps (kDenseLate) or lanes (kDenseTwo) were dense.
-constexpr int kDenseLate = 0, kDenseTwo = 1, kDenseTest = 2;
-
-template <int SB, int kDense, uint32_t kLutOff>
+// A step's state is a guess until the test for dense entries, after the next
+// step's entry read: a dense step is then looked up and its update, ring read
+// and the next entry read are redone.  The test and its branch (about 40
+// cycles) are off the chain; a redone step costs about 265 cycles.  kTwo (all
+// sub-blocks of the unit's tables in LDS): every step reads a second entry, the
+// dense lanes' from their sub-block, the others' their own again, which costs
+// about 75 cycles each step (only a 16-value sub-range can still be dense).
+// Returns how many steps were redone (kTwo: how many lanes were dense).
+// Batch-64 skew (256-value buckets, 40% of the steps dense): 92 -> 78 us with
+// kTwo and 8-step blocks.
+template <int SB, int NS, bool kWide, bool kTwo, uint32_t kLutOff>
 __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint32_t rn,
                                               uint32_t r2, uint32_t sub_addr, uint32_t& x,
                                               int& rp_io, uint32_t& esc) {
-  constexpr bool kWide = kDense != kDenseTest;
   constexpr int kB = kWide ? kWideBits : kLutBits;
-  constexpr bool kLate = kDense == kDenseLate;
+  constexpr bool kLate = !(kWide && kTwo);
   constexpr uint32_t kPos = (uint32_t)(DecGeom<SB>::kRing - 1);
   __attribute__((address_space(3))) uint32_t* recs = lds_ptr<uint32_t>(rec);
   auto entry_addr = [&](uint32_t tbase) {
@@ -2476,8 +2473,14 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
   u32x2 e0 = {0u, 0u};
   uint64_t dense = 0ull;
   auto redo = [&]() {
-    const uint64_t d = dense_lookup<true, kWide>(tb, ((uint64_t)e0.y << 32) | e0.x, x0 & 0xffffu,
-                                                 e0.y >= 0xffff0000u);
+    const bool dn = e0.y >= 0xffff0000u;
+    uint64_t d = ((uint64_t)e0.y << 32) | e0.x;
+    if constexpr (kTwo) {
+      if (dn) d = sub_entry<true>(tb, d, x0 & (kSubSize - 1));
+    } else {
+      d = dense_lookup<true, kWide>(tb, d, x0 & 0xffffu, dn);
+      ++dense_n;
+    }
     const StepUpdate n = step_update((uint32_t)d, (uint32_t)(d >> 32), x0, rp0 & kPos, 0u);
     const uint32_t w = *lds_ptr<uint16_t>(n.pos);
     const StepShadow h = step_shadow(n.m, (uint32_t)(d >> 32), n.up, rp0, r, esc0);
@@ -2485,10 +2488,9 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
     rp = h.rp;
     esc = h.esc;
     x = __builtin_amdgcn_perm(n.xn, w, h.sel);
-    ++dense_n;
   };
 #pragma unroll
-  for (int u = 0; u < SB; ++u) {
+  for (int u = 0; u < NS; ++u) {
     uint32_t addr = entry_addr(tbase);
     u32x2 e = *lds_ptr<u32x2>(addr + kLutOff);
     __builtin_amdgcn_sched_barrier(0);
@@ -2501,24 +2503,16 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
     if (u > 0) recs[(u - 1) * kLanes] = word;
     r = rn;
     rn = r2;
-    if (u + 2 < SB) r2 = recs[(u + 2) * kLanes];
-    if constexpr (kDense == kDenseTwo) {
-      // sub-block e.x, sub-range (cum >> 1) & 15
-      static_assert(kWideSubShift == 1 && kSubBits == 4 && kSubBytes == 128, "sub-block address");
-      const uint32_t sub = ((x << 2) & 0x78u) + sub_addr;
+    if (u + 2 < NS) r2 = recs[(u + 2) * kLanes];
+    if constexpr (kTwo) {
+      // sub-block e.x, sub-range (cum >> (12 - kB)) & 15
+      static_assert(kSubBits == 4 && kSubBytes == 128, "sub-block address");
+      constexpr int kShift = 16 - kB - kSubBits;
+      const uint32_t sub = ((kShift >= 3 ? x >> (kShift - 3) : x << (3 - kShift)) & 0x78u) + sub_addr;
       __builtin_amdgcn_sched_barrier(0);
       const bool dn = e.y >= 0xffff0000u;
       dense_n += (uint32_t)__popcll(ballot(dn));
       e = *lds_ptr<u32x2>((dn ? (e.x << 7) + sub : addr) + kLutOff);
-    }
-    if constexpr (kDense == kDenseTest) {
-      const bool dn = e.y >= 0xffff0000u;
-      if (__builtin_expect(ballot(dn) != 0ull, 0)) {
-        const uint64_t d =
-            dense_lookup<true, kWide>(tb, ((uint64_t)e.y << 32) | e.x, x & 0xffffu, dn);
-        e.x = (uint32_t)d;
-        e.y = (uint32_t)(d >> 32);
-      }
     }
     __builtin_amdgcn_sched_barrier(0);
     const StepUpdate n = step_update(e.x, e.y, x, rp & kPos, rn);
@@ -2540,7 +2534,7 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
     x = __builtin_amdgcn_perm(n.xn, w, h.sel);  // x << 16 | w, or x
   }
   if (kLate && __builtin_expect(dense != 0ull, 0)) redo();
-  recs[(SB - 1) * kLanes] = word;
+  recs[(NS - 1) * kLanes] = word;
   rp_io = uni((int)rp);
   return dense_n;
 }
@@ -2564,7 +2558,7 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
 // starts to the ring read, three LDS round trips; 16-step blocks fit beside
 // the tables since the records are 4 bytes).  P = 16: 94.7 -> 76.9 us, P = 4:
 // 29.9 -> 26.2 us.
-template <int SB, uint32_t kLutOff>
+template <int SB, int NS, uint32_t kLutOff>
 __device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, uint32_t rn,
                                                  uint32_t r2, int starts_off, uint32_t& x,
                                                  int& rp_io, uint32_t& esc) {
@@ -2597,7 +2591,7 @@ __device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, u
     return w;
   };
 #pragma unroll
-  for (int u = 0; u < SB; ++u) {
+  for (int u = 0; u < NS; ++u) {
     // entries of cum's 256-value bucket and of its 32-value part
     uint32_t ab, ap;
     asm("v_bfe_u32 %0, %2, 8, 8\n\tv_lshl_add_u32 %0, %0, 2, %3\n\t"
@@ -2609,7 +2603,7 @@ __device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, u
     __builtin_amdgcn_sched_barrier(0);
     r = rn;
     rn = r2;
-    if (u + 2 < SB) r2 = recs[(u + 2) * kLanes];
+    if (u + 2 < NS) r2 = recs[(u + 2) * kLanes];
     const uint32_t cum = x & 0xffffu, xh = x >> 16, c = x - 1u;
     const uint64_t fine = ballot((uint16_t)(cum + 1024u) < 2048u);  // cum < 1024 or >= 64512
     if (u > 0) recs[(u - 1) * kLanes] = word0();
@@ -2703,7 +2697,7 @@ __device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, u
     __builtin_amdgcn_sched_barrier(0);
     x = __builtin_amdgcn_perm(xn, w, sel);  // x << 16 | w, or x
   }
-  recs[(SB - 1) * kLanes] = word0();
+  recs[(NS - 1) * kLanes] = word0();
   rp_io = uni((int)rp);
 }
 
@@ -2807,30 +2801,39 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
   tb.lstarts = lstarts;
   const EarlyStage est = stage_early<kDecThreads, kLB, kSearch>(
       tb, llut, lclut, lstarts, a.tables, a.blob, a.M, a.starts_words, t_lo, t_hi, tid);
-  int32_t cbx[kPer], nbx[kPer];
-  float cm[kPer], nm[kPer];
-  auto load_block = [&](int j, int32_t* ib, float* im) {
+  // Per block parity, of the mapper's kPer steps: the block's inputs (ix: index
+  // or scale bits), loaded two blocks before they are mapped, and what the
+  // mapper keeps from mapping a block until it stores it (ko: the table's
+  // offset; ks: its symbol 0 and escape symbol << 16 as the coder has them; km:
+  // median or mean).  Two sets and a loop unrolled twice, not copies from one
+  // set to the other: a copy waits for the loads that were just issued.  Unit
+  // position p's byte offset is 4 (lane + 64 S (p / 64)); buffer accesses past
+  // the unit's last position read 0 and store nothing, so no branch goes around
+  // them (after one, the compiler waits for every outstanding access rather
+  // than for the oldest).  Batch-64 uniform: coder waits at the block barriers
+  // 137 -> 38 cycles per step, 83 -> 66 us.
+  int32_t ix[2][kPer];
+  const int64_t span =
+      len > 0 ? (int64_t)kLanes * (int64_t)a.S * (T - 1) + len - kLanes * (T - 1) : 0;
+  const __amdgpu_buffer_rsrc_t rin_i =
+      unit_rsrc(kMode == kModeGaussian ? (const void*)a.scales : (const void*)a.indexes,
+                row + start, kImplicit ? 0 : span);
+  const __amdgpu_buffer_rsrc_t rin_m =
+      unit_rsrc(a.means, row + start, kMode == kModeGaussian && a.means ? span : 0);
+  const int step_bytes = 4 * kLanes * (int)a.S;
+  auto load_block = [&](int j, int32_t* ib) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      const int u = (wid - 1) + kMappers * e;
-      if (SB % kMappers != 0 && u >= SB) break;
-      int p = lane + kLanes * (j * SB + u);
-      p = p < len ? p : len - 1;  // loads stay in the chunk; results are masked
-      const int32_t q = unit_pos(start, (int32_t)a.S, p);  // row position
-      if (kMode == kModeGaussian) {
-        ib[e] = __float_as_int(a.scales[row + q]);  // index found at map time
-        im[e] = a.means ? a.means[row + q] : 0.0f;
-      } else {
-        ib[e] = kImplicit ? 0 : a.indexes[row + q];
-        im[e] = kLatents ? a.medians[udiv((uint32_t)q, a.div_hw)] : 0.0f;
-      }
-    }
+    for (int e = 0; e < kPer; ++e)
+      ib[e] = kImplicit ? 0
+                        : (int32_t)__builtin_amdgcn_raw_buffer_load_b32(
+                              rin_i, 4 * lane + step_bytes * (j * SB + (wid - 1) + kMappers * e), 0,
+                              0);
   };
   // the mappers' first two blocks of inputs need neither the header checks
   // nor the tables
   if (wid != 0 && wid != kEscWave && nblk > 0) {
-    load_block(0, cbx, cm);
-    if (nblk > 1) load_block(1, nbx, nm);
+    load_block(0, ix[0]);
+    if (nblk > 1) load_block(1, ix[1]);
   }
   if (wid == 0) pc.mark_after_loads(1);  // header, offsets and metadata are in
   const bool hdr_ok = (hw[0] == kMagic) & (hw[1] == kVersion) & (hw[2] == a.B) &
@@ -2875,83 +2878,130 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
     const uint32_t* safe = reinterpret_cast<const uint32_t*>(cdata);
     q16 = (int)((cb - 4 * nst) / 2);
 
-    // Per mapped step, kept by its mapper until it stores the step two blocks
-    // later (o0, f0, m0: the block to store; o1, f1, m1: the one mapped last):
-    // the table's offset, its symbol 0 and escape symbol << 16 as the coder has
-    // them (s0, s1), and the median or mean.
-    uint32_t o0[kPer], o1[kPer], s0[kPer], s1[kPer];
-    float m0[kPer], m1[kPer];
+    uint32_t ko[2][kPer], ks[2][kPer];
+    float km[2][kPer];
+    const __amdgpu_buffer_rsrc_t rout =
+        unit_rsrc(kLatents ? (const void*)a.out_y : (const void*)a.out_sym, row + start, span);
 
-    // decoded values of block j -> HBM, escapes resolved first
-    auto store_block = [&](int j, bool last) {
-      const uint32_t* src = recs + (j & 1) * SB * kLanes;
-      const bool any_esc = uni((int)ctl[4 + (j & 1)]) != 0;
-      const uint32_t avail = (uint32_t)uni((int)ctl[1]);
+    // decoded values of block j (parity b) -> HBM, escapes resolved first
+    auto store_block = [&](int j, int b, bool last) __attribute__((always_inline)) {
+      const uint32_t* src = recs + b * SB * kLanes;
+      const bool any_esc = uni((int)ctl[4 + b]) != 0;
       uint32_t vals[kPer];
-      const uint32_t at = any_esc ? (uint32_t)uni((int)ctl[10 + (j & 1)]) : 0u;
 #pragma unroll
-      for (int e = 0; e < kPer; ++e) {
-        const int u = (wid - 1) + kMappers * e;
-        if (SB % kMappers != 0 && u >= SB) break;
-        const uint32_t word = src[u * kLanes + lane];  // the coder's
-        const uint32_t sym = word & 0xffffu;
-        uint32_t v = sym + o0[e] - (kSearch ? s0[e] & 0xffffu : 0u);
-        uint64_t em = 0;
-        if (any_esc) {  // the step's escaping lanes and its first escape entry
-          em = ballot(lane + kLanes * (j * SB + u) < len && sym == s0[e] >> 16);
+      for (int e = 0; e < kPer; ++e) vals[e] = src[((wid - 1) + kMappers * e) * kLanes + lane];
+      if (any_esc) {
+        const uint32_t avail = (uint32_t)uni((int)ctl[1]);
+        const uint32_t at = (uint32_t)uni((int)ctl[10 + b]);
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+          const int p = lane + kLanes * (j * SB + (wid - 1) + kMappers * e);
+          const uint32_t word = vals[e], sym = word & 0xffffu;
+          uint32_t v = sym + ko[b][e] - (kSearch ? ks[b][e] & 0xffffu : 0u);
+          // the step's escaping lanes and its first escape entry
+          const uint64_t em = ballot(p < len && sym == ks[b][e] >> 16);
           if (em)
-            esc_resolve<R>(em, at + (uint32_t)uni((int)(word >> 16)), o0[e], v, avail, fifo, enib,
-                           status, lane);
+            esc_resolve<R>(em, at + (uint32_t)uni((int)(word >> 16)), ko[b][e], v, avail, fifo,
+                           enib, status, lane);
+          if (!offsets_safe) {
+            const bool oob =
+                p < len && !((em >> lane) & 1ull) && (int32_t)v < (int32_t)ko[b][e];
+            status |= oob ? GAANS_ST_CORRUPT : 0u;
+            v = oob ? 0u : v;
+          }
+          vals[e] = v;
         }
-        // an ordinary symbol's value (sym < 2^16) overflows int32 exactly when
-        // it wraps below the offset
-        if (!offsets_safe) {
-          const bool oob = lane + kLanes * (j * SB + u) < len && !((em >> lane) & 1ull) &&
-                           (int32_t)v < (int32_t)o0[e];
-          status |= oob ? GAANS_ST_CORRUPT : 0u;
-          v = oob ? 0u : v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+          uint32_t v = (vals[e] & 0xffffu) + ko[b][e] - (kSearch ? ks[b][e] & 0xffffu : 0u);
+          // an ordinary symbol's value (its index < 2^16) overflows int32
+          // exactly when it wraps below the offset
+          if (!offsets_safe) {
+            const int p = lane + kLanes * (j * SB + (wid - 1) + kMappers * e);
+            const bool oob = p < len && (int32_t)v < (int32_t)ko[b][e];
+            status |= oob ? GAANS_ST_CORRUPT : 0u;
+            v = oob ? 0u : v;
+          }
+          vals[e] = v;
         }
-        vals[e] = v;
       }
       if (last) publish();
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
-        const int u = (wid - 1) + kMappers * e;
-        if (SB % kMappers != 0 && u >= SB) break;
-        const int p = lane + kLanes * (j * SB + u);
-        if (p < len) {
-          const int64_t i = row + unit_pos(start, (int32_t)a.S, p);
-          if (kLatents)
-            a.out_y[i] = __fadd_rn((float)(int32_t)vals[e], m0[e]);
-          else a.out_sym[i] = (int32_t)vals[e];
-        }
+        const int off = 4 * lane + step_bytes * (j * SB + (wid - 1) + kMappers * e);
+        const uint32_t v =
+            kLatents ? __float_as_uint(__fadd_rn((float)(int32_t)vals[e], km[b][e])) : vals[e];
+        __builtin_amdgcn_raw_buffer_store_b32(v, rout, off, 0, 0);
       }
     };
     GaussCoarse gc{};  // the mappers': the scale table's coarse level
-    auto map_block = [&](int j) {
-      uint32_t* dst = recs + (j & 1) * SB * kLanes;
+    auto map_block = [&](int j, int b) __attribute__((always_inline)) {
+      uint32_t* dst = recs + b * SB * kLanes;
+      int32_t t[kPer];
+      bool in = true;
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        if constexpr (kMode == kModeGaussian)
+          t[e] = gauss_index(__int_as_float(ix[b][e]), scl, a.n_scales, a.scales_pow2,
+                             a.scale_bound, gc);
+        else if constexpr (kImplicit)
+          t[e] = (int32_t)udiv((uint32_t)start +
+                                   (uint32_t)(lane + kLanes * (int)a.S *
+                                                         (j * SB + (wid - 1) + kMappers * e)),
+                               a.div_hw);
+        else t[e] = ix[b][e];
+        in = in & ((uint32_t)(t[e] - tb.t_lo) < (uint32_t)tb.nt);
+        // used when the block is stored, two turns on
+        if constexpr (kMode == kModeGaussian) {
+          km[b][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              rin_m, 4 * lane + step_bytes * (j * SB + (wid - 1) + kMappers * e), 0, 0));
+        } else if constexpr (kLatents) {
+          int p = lane + kLanes * (j * SB + (wid - 1) + kMappers * e);
+          p = p < len ? p : len - 1;  // the load stays in the medians
+          km[b][e] = a.medians[udiv((uint32_t)unit_pos(start, (int32_t)a.S, p), a.div_hw)];
+        }
+      }
+      if ((j + 1) * SB * kLanes <= len && ballot(!in) == 0ull) {
+        // every lane active, every table in LDS: no branch per step, all the
+        // metadata reads in flight together
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+          const uint4* lm = &tb.lmeta[t[e] - tb.t_lo];
+          ks[b][e] = lm->y;
+          ko[b][e] = lm->z;
+        }
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+          const int u = (wid - 1) + kMappers * e;
+          hash += index_term((uint32_t)(lane + kLanes * (j * SB + u)), (uint32_t)t[e]);
+          uint32_t r;
+          if constexpr (kSearch) {
+            r = search_record(tb, t[e], tb.lmeta[t[e]].x, ks[b][e], ks[b][e]);
+          } else {
+            ks[b][e] = (ks[b][e] - 1u) << 16;
+            r = (uint32_t)(t[e] - tb.t_lo) << (kWide ? kWideBits : kLutBits) | ks[b][e];
+          }
+          dst[u * kLanes + lane] = r;
+        }
+        return;
+      }
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
         const int u = (wid - 1) + kMappers * e;
-        if (SB % kMappers != 0 && u >= SB) break;
-        bool all_lds;
-        const int32_t ix = kMode == kModeGaussian
-                               ? gauss_index(__int_as_float(cbx[e]), scl, a.n_scales,
-                                             a.scales_pow2, a.scale_bound, gc)
-                               : cbx[e];
+        bool all_lds = true;
         uint32_t r;
         if constexpr (kSearch) {
-          r = dec_record_search(a, tb, lane, j * SB + u, len, ix, hash, status, o1[e], s1[e]);
-          all_lds = true;
+          r = dec_record_search(a, tb, lane, j * SB + u, len, t[e], hash, status, ko[b][e],
+                                ks[b][e]);
         } else {
-          r = dec_record<kImplicit, kWide>(a, tb, lane, j * SB + u, len, start, ix, hash,
-                                           status, all_lds, o1[e]);
-          s1[e] = r & 0xffff0000u;
+          r = dec_record<kWide>(a, tb, lane, j * SB + u, len, t[e], hash, status, all_lds,
+                                ko[b][e]);
+          ks[b][e] = r & 0xffff0000u;
         }
         dst[u * kLanes + lane] = r;
-        m1[e] = cm[e];
         if (!all_lds && lane == 0)
-          __hip_atomic_fetch_or(&ctl[2 + (j & 1)], 1u << u, __ATOMIC_RELAXED,
+          __hip_atomic_fetch_or(&ctl[2 + b], 1u << u, __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     };
@@ -2995,12 +3045,13 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
     if (wid == 0) {
       x = lane < A ? x : kStateLow;
       uint32_t ecur = 0;  // escape entries consumed
-      // Wide lookups: which way the next block's dense lanes go, by how many
-      // the last one had (a channel's table decides, and a chunk's channels
-      // differ).  kDenseTwo costs what kDenseLate does at three dense steps in
-      // ten.  sub_addr: LDS address of sub-block 0 of the blob, less kFixed.
-      const bool two_ok = kWide && bd.d1 > bd.d0 && tb.sub_n == bd.d1 - bd.d0;
-      bool two = false;
+      // Whether the next block reads two entries per step, by how many dense
+      // steps the last one had (a channel's table decides, and a chunk's
+      // channels differ): that costs what three redone steps in ten do.
+      // sub_addr: LDS address of sub-block 0 of the blob, less kFixed.
+      const bool two_ok = !kSearch && bd.d1 > bd.d0 && tb.sub_n == bd.d1 - bd.d0;
+      // (256-value buckets begin with two: half of most tables' steps are dense)
+      bool two = !kWide && two_ok;
       const uint32_t sub_addr = (uint32_t)((kLutEntry * kLB + 16) * a.nt_cap) -
                                 (uint32_t)kSubBytes * tb.sub_first;
       // The coder's chain of dependent steps bounds the block loop; its
@@ -3018,31 +3069,47 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
         const uint32_t nl = kSearch ? 0u : (uint32_t)uni((int)ctl[2 + (j & 1)]);
         if (!kSearch) ctl[2 + (j & 1)] = 0u;  // every lane: no exec-mask branch
         uint32_t esc = 0u;  // escapes of the block
+        const uint32_t rec =
+            (uint32_t)G::kRingBytes + 4u * (uint32_t)((j & 1) * SB * kLanes + lane);
+        constexpr uint32_t kLut = (uint32_t)G::kFixed;
         if ((j + 1) * SB * kLanes <= len && nl == 0) {
           // common case: every lane of the block active, LDS tables
-          if constexpr (kSearch) {
-            dec_block_search<SB, (uint32_t)G::kFixed>(
-                tb, (uint32_t)G::kRingBytes + 4u * (uint32_t)((j & 1) * SB * kLanes + lane), rn,
-                r2, starts_off, x, rp, esc);
-          } else {
-            const uint32_t rec =
-                (uint32_t)G::kRingBytes + 4u * (uint32_t)((j & 1) * SB * kLanes + lane);
-            constexpr uint32_t kLut = (uint32_t)G::kFixed;
-            if constexpr (!kWide) {
-              dec_block<SB, kDenseTest, kLut>(tb, rec, rn, r2, 0u, x, rp, esc);
-            } else if (two) {
-              two = dec_block<SB, kDenseTwo, kLut>(tb, rec, rn, r2, sub_addr, x, rp, esc) * 4u >=
-                    (uint32_t)SB;
+          if constexpr (kSearch)
+            dec_block_search<SB, SB, kLut>(tb, rec, rn, r2, starts_off, x, rp, esc);
+          else if (two)
+            two = dec_block<SB, SB, kWide, true, kLut>(tb, rec, rn, r2, sub_addr, x, rp, esc) *
+                      4u >=
+                  (uint32_t)SB;
+          else
+            two = dec_block<SB, SB, kWide, false, kLut>(tb, rec, rn, r2, 0u, x, rp, esc) * 10u >=
+                      3u * (uint32_t)SB &&
+                  two_ok;
+        } else {
+          // the last block, or tables outside LDS: its full steps four and one
+          // at a time, then the rest
+          const int n = T - j * SB < SB ? T - j * SB : SB;
+          const int full = nl ? 0 : (len / kLanes - j * SB < n ? len / kLanes - j * SB : n);
+          int u = 0;
+          while (u < full) {
+            const uint32_t at = rec + 4u * (uint32_t)(u * kLanes);
+            const uint32_t ra = src[u * kLanes + lane];
+            if (u + 4 <= full) {
+              const uint32_t rb = src[(u + 1) * kLanes + lane];
+              if constexpr (kSearch)
+                dec_block_search<SB, 4, kLut>(tb, at, ra, rb, starts_off, x, rp, esc);
+              else if (two)
+                dec_block<SB, 4, kWide, true, kLut>(tb, at, ra, rb, sub_addr, x, rp, esc);
+              else dec_block<SB, 4, kWide, false, kLut>(tb, at, ra, rb, 0u, x, rp, esc);
+              u += 4;
             } else {
-              two = dec_block<SB, kDenseLate, kLut>(tb, rec, rn, r2, 0u, x, rp, esc) * 10u >=
-                        3u * (uint32_t)SB &&
-                    two_ok;
+              if constexpr (kSearch)
+                dec_block_search<SB, 1, kLut>(tb, at, ra, ra, starts_off, x, rp, esc);
+              else dec_block<SB, 1, kWide, false, kLut>(tb, at, ra, ra, 0u, x, rp, esc);
+              ++u;
             }
           }
-        } else {
-          // last block or tables outside LDS: one step at a time
 #pragma unroll 1
-          for (int u = 0; u < SB && j * SB + u < T; ++u) {
+          for (; u < n; ++u) {
             const uint32_t ru = src[u * kLanes + lane];
             const bool act = lane + kLanes * (j * SB + u) < len;
             uint32_t v;
@@ -3086,30 +3153,26 @@ __global__ __launch_bounds__(kDecThreads, kDecWavesPerSimd) void k_decode(DecArg
       __syncthreads();
     } else {
       if (kMode == kModeGaussian) gc = gauss_coarse(scl, a.n_scales);  // staged, published
-      if (nblk > 0) map_block(0);
+      if (nblk > 0) map_block(0, 0);
+      if (nblk > 2) load_block(2, ix[0]);
       __syncthreads();
-      for (int j = 0; j < nblk; ++j) {
-        // mappers: store block j - 1 and map block j + 1 while the coder decodes block j
-        if (j > 0) store_block(j - 1, false);
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) {
-          o0[e] = o1[e];
-          s0[e] = s1[e];
-          m0[e] = m1[e];
-        }
+      // while the coder decodes block j: store block j - 1 and map block j + 1
+      // (both of parity b), then load block j + 3
+      auto turn = [&](int j, int b) __attribute__((always_inline)) {
+        if (j > 0) store_block(j - 1, b, false);
         if (j + 1 < nblk) {
-#pragma unroll
-          for (int e = 0; e < kPer; ++e) {
-            cbx[e] = nbx[e];
-            cm[e] = nm[e];
-          }
-          if (j + 2 < nblk) load_block(j + 2, nbx, nm);
-          map_block(j + 1);
+          map_block(j + 1, b);
+          if (j + 3 < nblk) load_block(j + 3, ix[b]);
         }
         __syncthreads();
+      };
+      for (int j = 0; j < nblk; j += 2) {
+        turn(j, 1);
+        if (j + 1 < nblk) turn(j + 1, 0);
       }
-      if (nblk > 0) store_block(nblk - 1, true);
-      else publish();
+      if (nblk == 0) publish();
+      else if (nblk & 1) store_block(nblk - 1, 0, true);
+      else store_block(nblk - 1, 1, true);
       __syncthreads();
     }
   }
@@ -3545,15 +3608,14 @@ struct Stage {
   int32_t nt_cap, ne_cap, nd_cap, stage_all;
 };
 
-// LDS of one workgroup when occ workgroups share a CU: the CU's LDS divided
-// by occ, rounded down to 1 KB, less 1 KB when several share it (measured on
-// MI355X: three workgroups of 53,632 bytes fit on a CU, three of 54,272 do
+// LDS of one workgroup when occ workgroups share a CU.  gfx950 allocates a
+// CU's 160 KB in 128 units of 1,280 bytes (measured: three workgroups of
+// 53,632 and of 53,760 = 42 x 1,280 bytes fit on a CU, three of 54,272 do
 // not).
 int64_t lds_budget(const DevLds& d, int64_t occ) {
-  int64_t b = d.per_cu / occ;
-  if (b > d.per_block) b = d.per_block;
-  b = b / 1024 * 1024;
-  return occ > 1 ? b - 1024 : b;
+  const int64_t unit = d.per_cu / 128;
+  const int64_t b = 128 / occ * unit;
+  return b > d.per_block ? d.per_block : b;
 }
 
 // Workgroups per CU that keep a launch of units workgroups in one round.
@@ -3627,12 +3689,13 @@ EncPlan plan_encode(const gaans_tables* t, int64_t P, int64_t units, const DevLd
 // Decoder: lookups and metadata per table; sub-blocks when they are staged
 // too.  For each workgroups-per-CU count (at most 3: the kernel is built for
 // 6 waves per SIMD, and a 6-wave workgroup puts two waves on two of the CU's
-// four SIMDs), the options in order of preference: 8-step blocks with
-// sub-blocks, 4-step blocks with sub-blocks (their records, stream ring and
-// escape FIFO take half the LDS); then, when the blob has them and every
+// four SIMDs), the options in order of preference, each with 16-, 8-, then
+// 4-step blocks (their records, stream ring and escape FIFO halve): the lookups
+// with room for every unit's sub-blocks; then, when the blob has them and every
 // position may use any table (explicit or computed indexes), the search
-// lookups of all tables; then the lookups without sub-blocks (a dense-bucket
-// lookup then reads global memory).
+// lookups of all tables; then the lookups with the sub-blocks that fit, if that
+// is 1.25 times a typical range's (16 x 320 x 17 x 31, P = 8: 36.9 -> 32.9 us);
+// then without sub-blocks (a dense-bucket lookup then reads global memory).
 struct DecPlan {
   Stage st;
   int sb;
@@ -3687,10 +3750,21 @@ DecPlan plan_decode(const gaans_tables* t, int64_t P, int64_t units, const DevLd
                        (size_t)(fixed + per_wide * s.nt_cap + kSubBytes * (int64_t)s.nd_cap),
                        false, 0, true};
       }
-    for (int opt = 0; opt < 9; ++opt) {
+    const int64_t typical_d = (P * t->total_dense + t->M - 1) / t->M * 5 / 4;
+    for (int opt = 0; opt < 12; ++opt) {
       const int sb = 16 >> (opt % 3);  // 16-, 8-, then 4-step blocks of each kind
       const int64_t fixed = dec_fixed_lds(sb);
       if (opt >= 3 && !has_dense) break;  // same as the options already tried
+      if (opt >= 6 && opt < 9) {  // as many sub-blocks as the rest of the LDS holds
+        Stage s;
+        if (sb < 8 || !fit_stage(t, P, per_table, 0, 0, cap - fixed - extra, &s, range_ok)) continue;
+        const int64_t room = (cap - fixed - extra - per_table * s.nt_cap) / kSubBytes;
+        if (room < typical_d || room < 1) continue;
+        s.nd_cap = (int32_t)(room < (int64_t)t->total_dense ? room : t->total_dense);
+        return DecPlan{s, sb,
+                       (size_t)(fixed + per_table * s.nt_cap + kSubBytes * (int64_t)s.nd_cap),
+                       false, 0, false};
+      }
       if (opt >= 3 && opt < 6) {
         if (search_ok && fixed + search_bytes + extra <= cap)
           return DecPlan{Stage{(int32_t)t->M, 0, 0, 1}, sb, (size_t)(fixed + search_bytes), true,
