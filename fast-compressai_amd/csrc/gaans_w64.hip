@@ -276,7 +276,9 @@ struct Tabs {
   const uint2* __restrict__ gent;
   const uint64_t* __restrict__ glut;
   const uint64_t* __restrict__ gsub;
-  const uint4* lmeta;      // {ent_base (LDS-local), nsym, offset, ent_base (global)}
+  // decoder: {ent_base (LDS-local), nsym, offset, ent_base (global)}; encoder:
+  // {LDS address of symbol 0's entry, nsym - 1, offset, unused}
+  const uint4* lmeta;
   const uint2* lent;       // encoder: both entry words
   const uint64_t* llut;    // decoder: nt x 256 (wide: nt x kWideSize) lookup entries
   const uint64_t* lsub;    // decoder: sub-blocks of the staged tables
@@ -314,11 +316,11 @@ __device__ __forceinline__ void copy16_dma(uint4* dst, const uint4* __restrict__
   }
 }
 
-template <int NT, bool kEnt, bool kSub>
+template <int NT, bool kEnt, bool kSub, bool kEncMeta = false>
 __device__ __forceinline__ void stage_pass(const Tabs& T, uint4* lmeta, uint2* lent, uint4* lsub,
                                            const uint4* __restrict__ ssrc, uint32_t nt,
                                            uint32_t ne, uint32_t nd, uint32_t base0, int t_lo,
-                                           int tid) {
+                                           int tid, uint32_t lent_addr = 0u) {
   // loads in flight per thread and kind (fewer for the decoder's larger
   // workgroup, whose waves keep more registers live across the staging)
   constexpr int U = NT >= 384 ? 3 : 4;
@@ -340,7 +342,10 @@ __device__ __forceinline__ void stage_pass(const Tabs& T, uint4* lmeta, uint2* l
     for (int k = 0; k < U; ++k) {
       const uint32_t i = b + k * NT;
       lmeta[i < nt ? i : nt - 1] =
-          make_uint4(mv[k].ent_base - base0, mv[k].nsym, (uint32_t)mv[k].offset, mv[k].ent_base);
+          kEncMeta ? make_uint4(lent_addr + 8u * (mv[k].ent_base - base0), mv[k].nsym - 1u,
+                                (uint32_t)mv[k].offset, 0u)
+                   : make_uint4(mv[k].ent_base - base0, mv[k].nsym, (uint32_t)mv[k].offset,
+                                mv[k].ent_base);
       if (kEnt) lent[i < ne ? i : ne - 1] = ev[k];
       if (kSub) lsub[i < nd ? i : nd - 1] = dv[k];
     }
@@ -390,7 +395,8 @@ __device__ __forceinline__ StageBounds stage_bounds_wide(const uint32_t* __restr
 // LB: lookup entries per table (kLutSize, or kWideSize for the wide lookups)
 template <int NT, int LB = kLutSize>
 __device__ void stage_tables(Tabs& T, uint4* lmeta, uint2* lent, uint64_t* llut, uint64_t* lsub,
-                             const StageBounds& bd, int t_lo, int t_hi, int tid) {
+                             const StageBounds& bd, int t_lo, int t_hi, int tid,
+                             uint32_t lent_addr = 0u) {
   T.t_lo = t_lo;
   T.nt = t_hi > t_lo ? t_hi - t_lo : 0;
   T.sub_first = 0;
@@ -407,7 +413,8 @@ __device__ void stage_tables(Tabs& T, uint4* lmeta, uint2* lent, uint64_t* llut,
       copy16_dma<NT>(reinterpret_cast<uint4*>(lent),
                      reinterpret_cast<const uint4*>(T.gent + b2), (bd.ent_end - b2 + 1u) / 2u,
                      tid);
-      stage_pass<NT, false, false>(T, lmeta, nullptr, nullptr, nullptr, nt, 1u, 0u, b2, t_lo, tid);
+      stage_pass<NT, false, false, true>(T, lmeta, nullptr, nullptr, nullptr, nt, 1u, 0u, b2, t_lo,
+                                         tid, lent_addr);
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's direct-to-LDS copies are in
     } else {
       // lookups and sub-blocks straight into LDS, the metadata rows through
@@ -703,10 +710,10 @@ __device__ void unit_end_offsets(const EncArgs& a, int tid, uint64_t* sh) {
 }
 
 // Op record of one lane and step (16 bytes):
-//   x: start | (65536 - freq) << 16      (identity op: 0)
-//   y: division magic of freq            (enc_div)
-//   z: shift (enc_shift) | escape << 8 | (freq - 1) << 16
-//      (identity op: 15 | 0xffff << 16, so that it never emits)
+//   x: entry word 0, start | (freq - 1) << 16   (identity op: 0xffff << 16,
+//      which never emits and adds nothing)
+//   y: division magic of freq                   (enc_div)
+//   z: shift (enc_shift) | escape << 8
 //   w: escape raw value
 // CompressAI's escape split (reference warp_ans_kernel_v2.cu:139-164):
 // v = sym - offset; v < 0 -> raw = -2v - 1, v >= maxv -> raw = 2 (v - maxv),
@@ -753,7 +760,7 @@ __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, in
     if (kLds) {
       const uint4 m = tb.lmeta[tbi - tb.t_lo];
       ebase[e] = m.x;
-      nsym[e] = m.y;
+      nsym[e] = m.y + 1u;
       offset[e] = (int32_t)m.z;
     } else {
       const TabMeta m = tb.gmeta[tbi];
@@ -772,8 +779,13 @@ __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, in
     ovf[e] = ((sym[e] ^ offset[e]) & (sym[e] ^ v[e])) < 0;
     const bool out = ((uint32_t)v[e] >= (uint32_t)maxv) | ovf[e];
     esc[e] = ok[e] & out;
-    const uint32_t at = ebase[e] + (uint32_t)(out ? maxv : v[e]);
-    ent[e] = kLds ? tb.lent[at] : tb.gent[at];
+    const uint32_t i = (uint32_t)(out ? maxv : v[e]);
+    if constexpr (kLds) {
+      const u32x2 w = *lds_ptr<u32x2>(ebase[e] + 8u * i);
+      ent[e] = make_uint2(w.x, w.y);
+    } else {
+      ent[e] = tb.gent[ebase[e] + i];
+    }
   }
 #pragma unroll
   for (int e = 0; e < KP; ++e) {
@@ -790,9 +802,9 @@ __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, in
     const uint32_t fr = (ent[e].x >> 16) + 1u;
     const uint32_t sh = enc_shift(fr);
     uint4 r;
-    r.x = ok[e] ? ((ent[e].x & 0xffffu) | ((65536u - fr) << 16)) : 0u;
+    r.x = ok[e] ? ent[e].x : 0xffff0000u;
     r.y = ok[e] ? ent[e].y : 1u;
-    r.z = (ok[e] ? sh | (ent[e].x & 0xffff0000u) : 0xffff000fu) | (esc[e] ? 256u : 0u);
+    r.z = (ok[e] ? sh : 0u) | (esc[e] ? 256u : 0u);
     r.w = raw;
     rec[e] = r;
   }
@@ -807,10 +819,9 @@ __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, in
 // when a lane of the block has an index outside the staged tables or a value
 // outside int32 (the caller then maps the block with enc_records); else sets
 // bit e of esc_steps for each step e with an escape.
-//   x = start | (65535 - (freq - 1)) << 16 = entry word 0 ^ 0xffff0000
-//   z = 31 - ffbh(freq - 1): the shift for freq >= 2, and 32 (the freq-1
-//       flag) for freq = 1, where ffbh(0) = 0xffffffff; | 256 for an escape;
-//       | (freq - 1) << 16 = entry word 0's high half
+//   z = enc_shift: the bits of freq - 1, entry word 0's high half: 16 less the
+//       word's leading zeros, and 0 for freq = 1, whose word has at least 16
+//       (none set, start = 0: 0xffffffff)
 template <int kMode, bool kImplicit, int KP>
 __device__ __forceinline__ bool enc_records_fast(const EncArgs& a, const Tabs& tb, int lane,
                                                  int t0, int tstep, int32_t start,
@@ -845,21 +856,18 @@ __device__ __forceinline__ bool enc_records_fast(const EncArgs& a, const Tabs& t
   for (int e = 0; e < KP; ++e) {
     const uint4 m = tb.lmeta[tbl[e] - tb.t_lo];
     v[e] = (uint32_t)sym[e] - m.z;
-    maxv[e] = m.y - 1u;
+    maxv[e] = m.y;
     off[e] = m.z;
-    const bool out = v[e] >= maxv[e];
-    om[e] = ballot(out);
-    at[e] = m.x + (out ? maxv[e] : v[e]);
+    om[e] = ballot(v[e] >= maxv[e]);
+    at[e] = m.x + 8u * (v[e] < maxv[e] ? v[e] : maxv[e]);
   }
   uint32_t es = 0;
 #pragma unroll
   for (int e = 0; e < KP; ++e) {
-    const uint2 ent = tb.lent[at[e]];
-    // enc_shift: 31 - clz(2 (freq - 1) + 1) (never of zero), from the
-    // entry's (freq - 1) << 16 | start
-    uint32_t lz;
-    asm("v_ffbh_u32 %0, %1" : "=v"(lz) : "v"((ent.x >> 15) | 1u));
-    rec[e] = make_uint4(ent.x ^ 0xffff0000u, ent.y, (31u - lz) | (ent.x & 0xffff0000u), 0u);
+    const u32x2 ent = *lds_ptr<u32x2>(at[e]);
+    uint32_t sh;
+    asm("v_ffbh_u32 %0, %1\n\tv_sub_u16_e64 %0, 16, %0 clamp" : "=v"(sh) : "v"(ent.x));
+    rec[e] = make_uint4(ent.x, ent.y, sh, 0u);
     if (om[e] != 0ull) {
       // the escape split of enc_records for this step's escaping lanes
       const bool esc = (om[e] >> lane) & 1ull;
@@ -903,33 +911,112 @@ __device__ __forceinline__ void ring_flush(uint16_t* __restrict__ wbuf, const ui
   for (int i = (a0 >> 2) + lane; i < (a1 >> 2); i += kLanes) w64[i] = r64[(uint32_t)i & m64];
 }
 
-// The ring holds the words [wp, fl) (positions mod the ring size).  The coder
-// flushes it at the start of a block when fewer than SB * kLanes slots are
-// free (a step emits at most one word per lane), so the steps need no check.
-// A lane emits when x >= freq << 16, i.e. (x >> 16) > freq - 1 (z's high
-// half): one compare of the two high halves.  Every lane stores, the ones
-// that emit nothing to their spare slot (spare = ring_mask + 1 + lane,
-// computed once per wave): selects on the compare rather than an
-// exec-masked branch, which costs three scalar instructions more per step
-// and keeps consecutive steps from interleaving.  (With the spare slot
-// computed here the compiler turned the selects back into a branch.)
-__device__ __forceinline__ void emit_words(uint32_t z, uint32_t& x, uint16_t* ring, int& wp,
-                                           uint32_t spare, uint32_t ring_mask) {
-  const bool emit = (x >> 16) > (z >> 16);
-  const uint64_t m = ballot(emit);
-  wp = uni(wp - __popcll(m));
-  // wp + the number of emitting lanes below this one
-  const uint32_t pos = (uint32_t)__builtin_amdgcn_mbcnt_hi(
-      (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)wp));
-  ring[emit ? pos & ring_mask : spare] = (uint16_t)x;
-  x = emit ? x >> 16 : x;
-}
+// Steps NS - 1 .. 0 of the coder.  rec: LDS address of the lane's record of
+// step 0 (the next steps' are 16 kLanes bytes apart).  n = -wp, the same in
+// every lane: the ring holds the words [wp, fl) (positions mod the ring size,
+// mask = ring words - 1, ring at LDS address 0).  The coder flushes it at the
+// start of a block when fewer than SB * kLanes slots are free (a step emits at
+// most one word per lane), so the steps need no check.
+//
+// A lane emits when x >= freq << 16, i.e. (x >> 16) > freq - 1: one compare of
+// the two high halves; y = x >> 16 or x is then coded as x' = ((y / freq) <<
+// 16) + y % freq + start = y + start + q (65536 - freq), q = (mulhi(y, m) + y)
+// >> l (enc_div; for freq = 1 too: q = y < 2^16).  Every lane stores, the ones
+// that emit nothing to their spare slot (ring words + lane): selects on the
+// compare, no exec-masked branch.
+//
+// The step is bound by its issue slots, one per four cycles and more: 14 or 15
+// vector operations, the record read two steps ahead and the store of the step
+// before, which keep the wait states between the compare and its readers.
+// kScalar: the words are counted by a scalar bit count, two vector operations
+// fewer, but the chain waits for it; without, by vector ones.  With one
+// workgroup per CU the coder's wave has slots to spare and the wait counts
+// (lone wave 130 -> 93 cycles per step; 2160x3840 symbols 91 -> 79 us); with
+// several per CU the SIMDs' vector slots are full (batch-64 uniform 68 -> 74 us
+// with the vector counts).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// main rANS op: x' = ((x / freq) << 16) + x % freq + start = x + start + q (65536 - freq)
-// (for freq = 1 too: q = x < 2^16, x' = x 2^16 + start)
-__device__ __forceinline__ uint32_t enc_apply(uint32_t x, uint4 r) {
-  const uint32_t q = enc_div(x, r.y, r.z);
-  return __umul24(q, r.x >> 16) + x + (r.x & 0xffffu);
+// kz, kw: the records' z and w are kept there (kKeep: the coder lists the
+// escapes).
+template <int NS, bool kScalar, bool kKeep>
+__device__ __forceinline__ void enc_steps(uint32_t rec, uint32_t spare, uint32_t mask, uint32_t& x,
+                                          uint32_t& n, int& wp, uint32_t* kz, uint32_t* kw) {
+  __attribute__((address_space(3))) u32x4* recs = lds_ptr<u32x4>(rec);
+  u32x4 r1 = recs[(NS - 1) * kLanes], r2 = r1;
+  if (NS > 1) r2 = recs[(NS - 2) * kLanes];
+  uint32_t at0 = 0u, x0 = 0u;  // the step before: its store's address and word
+#pragma unroll
+  for (int k = NS - 1; k >= 0; --k) {
+    const u32x4 r = r1;
+    r1 = r2;
+    uint32_t f;  // 65536 - freq
+    register uint64_t m asm("vcc");
+    asm("v_cmp_gt_u32_sdwa vcc, %[x], %[rx] src0_sel:WORD_1 src1_sel:WORD_1\n\t"
+        "v_xor_b32_sdwa %[f], %[low], %[rx] dst_sel:DWORD dst_unused:UNUSED_PAD "
+        "src0_sel:DWORD src1_sel:WORD_1"
+        : [f] "=&v"(f), "=s"(m)
+        : [x] "v"(x), [rx] "v"(r.x), [low] "v"(0xffffu));
+    __builtin_amdgcn_sched_barrier(0);
+    if (k >= 2) r2 = recs[(k - 2) * kLanes];
+    if (k < NS - 1) *lds_ptr<uint16_t>(at0) = (uint16_t)x0;
+    __builtin_amdgcn_sched_barrier(0);
+    if (NS == 1 || (NS == 2 && k == 1)) asm volatile("s_nop 0" : "+s"(m));  // neither of the two
+    uint32_t y, q, b, at, xn;
+    if constexpr (kScalar) {
+      wp -= __popcll(m);
+      asm("v_cndmask_b32_sdwa %[y], %[x], %[x], vcc dst_sel:DWORD dst_unused:UNUSED_PAD "
+          "src0_sel:DWORD src1_sel:WORD_1\n\t"
+          "v_mov_b32_e32 %[at], %[wp]\n\t"
+          "v_mul_hi_u32 %[q], %[y], %[m]\n\t"
+          "v_mbcnt_lo_u32_b32 %[at], vcc_lo, %[at]\n\t"
+          "v_add_u32_e32 %[q], %[q], %[y]\n\t"
+          "v_mbcnt_hi_u32_b32 %[at], vcc_hi, %[at]\n\t"
+          "v_lshrrev_b32_e32 %[q], %[z], %[q]\n\t"
+          "v_and_b32_e32 %[at], %[mask], %[at]\n\t"
+          "v_add_u32_sdwa %[b], %[y], %[rx] dst_sel:DWORD dst_unused:UNUSED_PAD "
+          "src0_sel:DWORD src1_sel:WORD_0\n\t"
+          "v_cndmask_b32_e32 %[at], %[spare], %[at], vcc\n\t"
+          "v_mad_u32_u24 %[xn], %[q], %[f], %[b]\n\t"
+          "v_lshlrev_b32_e32 %[at], 1, %[at]"
+          : [y] "=&v"(y), [q] "=&v"(q), [b] "=&v"(b), [at] "=&v"(at), [xn] "=&v"(xn), "+s"(m)
+          : [x] "v"(x), [z] "v"(r.z), [rx] "v"(r.x), [m] "v"(r.y), [f] "v"(f), [wp] "s"(wp),
+            [mask] "s"(mask), [spare] "v"(spare),
+            // not read: keeps the compiler from giving its register, which the
+            // record read in flight writes, to y, and waiting for that read
+            "v"(r.w));
+    } else {
+      uint32_t n1;
+      asm("v_cndmask_b32_sdwa %[y], %[x], %[x], vcc dst_sel:DWORD dst_unused:UNUSED_PAD "
+          "src0_sel:DWORD src1_sel:WORD_1\n\t"
+          "v_bcnt_u32_b32 %[n1], vcc_lo, %[n]\n\t"
+          "v_mbcnt_lo_u32_b32 %[at], vcc_lo, 0\n\t"
+          "v_mul_hi_u32 %[q], %[y], %[m]\n\t"
+          "v_bcnt_u32_b32 %[n1], vcc_hi, %[n1]\n\t"
+          "v_mbcnt_hi_u32_b32 %[at], vcc_hi, %[at]\n\t"
+          "v_add_u32_e32 %[q], %[q], %[y]\n\t"
+          "v_sub_u32_e32 %[at], %[at], %[n1]\n\t"
+          "v_lshrrev_b32_e32 %[q], %[z], %[q]\n\t"
+          "v_and_b32_e32 %[at], %[mask], %[at]\n\t"
+          "v_add_u32_sdwa %[b], %[y], %[rx] dst_sel:DWORD dst_unused:UNUSED_PAD "
+          "src0_sel:DWORD src1_sel:WORD_0\n\t"
+          "v_cndmask_b32_e32 %[at], %[spare], %[at], vcc\n\t"
+          "v_mad_u32_u24 %[xn], %[q], %[f], %[b]\n\t"
+          "v_lshlrev_b32_e32 %[at], 1, %[at]"
+          : [y] "=&v"(y), [q] "=&v"(q), [b] "=&v"(b), [at] "=&v"(at), [xn] "=&v"(xn),
+            [n1] "=&v"(n1), "+s"(m)
+          : [x] "v"(x), [z] "v"(r.z), [rx] "v"(r.x), [m] "v"(r.y), [f] "v"(f), [n] "v"(n),
+            [mask] "s"(mask), [spare] "v"(spare), "v"(r.w));  // r.w: as above
+      n = n1;
+    }
+    if constexpr (kKeep) {
+      kz[k] = r.z;
+      kw[k] = r.w;
+    }
+    at0 = at;
+    x0 = x;
+    x = xn;
+  }
+  *lds_ptr<uint16_t>(at0) = (uint16_t)x0;
 }
 
 // Escapes of one step into the unit's escape list: slots are taken from the
@@ -1257,13 +1344,11 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
   constexpr int kWaves = G::kWaves, kThreads = G::kThreads;
   constexpr int kPer = G::kPer;
   // Who lists the escapes: with eight mappers (a CU to each workgroup) the
-  // first mapper wave, off the coder's chain (2160x3840 latent encode 95 ->
-  // 89 us, hyperprior y 45 -> 44 us at P=16); else the coder, since with
-  // four mappers and several workgroups per CU the mappers have no time to
-  // spare (batch-64 uniform 67 -> 72 us with the listing moved), and the
-  // latents' mappers, which quantize, neither (512x768 latent 17.7 -> 18.1
-  // us).
-  constexpr bool kMList = NM == 8 && kMode != kModeLatents;
+  // first mapper wave, off the coder's chain (2160x3840 latents with 16-step
+  // blocks 94 -> 80 us); else the coder, since with four mappers and several
+  // workgroups per CU the mappers have no time to spare (batch-64 uniform 67
+  // -> 72 us with the listing moved).
+  constexpr bool kMList = NM == 8;
   extern __shared__ __align__(16) uint8_t smem[];
   uint16_t* ring = reinterpret_cast<uint16_t*>(smem);
   const uint32_t ring_mask = a.ring_mask;  // ring words - 1
@@ -1359,8 +1444,14 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
   tb.lsub = nullptr;
   // mapper wave w (1..kEncMappers) owns steps u = w - 1 + kEncMappers e of every block
   // (steps a wave does not own keep these zeros)
-  int32_t ca[kPer] = {}, cb[kPer] = {}, na[kPer] = {}, nb[kPer] = {};
-  float cm[kPer] = {}, nm[kPer] = {};
+  // Inputs of two blocks, by the parity of the block's turn (block nblk - 1 is
+  // turn 0): two sets and a loop unrolled twice, not copies from one to the
+  // other, which would wait for the loads that were just issued.  A block
+  // before the first loads nothing (its offsets are out of range), so the loads
+  // need no condition: after one, the compiler waits for every outstanding load
+  // instead of counting.
+  int32_t ia[2][kPer] = {}, ib[2][kPer] = {};
+  float im[2][kPer] = {};
   // The unit's inputs as buffer resources over its len positions: a load's
   // address is the lane's constant byte offset plus the step's (one add, no
   // 64-bit address arithmetic per load), and lanes past the unit's end read
@@ -1378,7 +1469,7 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
   const __amdgpu_buffer_rsrc_t rin_m = unit_rsrc(has_m ? (const void*)a.means : in_a_ptr,
                                                  row + start, has_m ? span : 0);
   const int lane4 = 4 * lane;
-  auto load_block = [&](int j, int32_t* ia, int32_t* ib, float* im) __attribute__((always_inline)) {
+  auto load_block = [&](int j, int32_t* va, int32_t* vb, float* vm) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < kPer; ++e) {
       const int u = (wid - 1) + kEncMappers * e;
@@ -1386,28 +1477,28 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       // the range check covers the vector offset only (not a scalar one),
       // so the step's offset is added to the lane's
       const int vo = lane4 + uni(4 * kLanes * a.S * (j * SB + u));
-      ia[e] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rin_a, vo, 0, 0);
+      va[e] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rin_a, vo, 0, 0);
       if (kMode == kModeGaussian) {
-        im[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rin_m, vo, 0, 0));
+        vm[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rin_m, vo, 0, 0));
         // the index is found from the scale when the block is mapped
-        ib[e] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rin_b, vo, 0, 0);
+        vb[e] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rin_b, vo, 0, 0);
       } else {
         if (kMode == kModeLatents) {
-          int p = lane + kLanes * (j * SB + u);
-          p = p < len ? p : len - 1;  // the median's channel stays in the chunk
-          im[e] = a.medians[udiv((uint32_t)unit_pos(start, a.S, p), a.div_hw)];
+          uint32_t p = (uint32_t)(lane + kLanes * (j * SB + u));
+          p = p < (uint32_t)len ? p : (uint32_t)len - 1u;  // the channel stays in the chunk
+          vm[e] = a.medians[udiv((uint32_t)unit_pos(start, a.S, (int)p), a.div_hw)];
         } else {
-          im[e] = 0.0f;
+          vm[e] = 0.0f;
         }
-        ib[e] = kImplicit ? 0 : (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rin_b, vo, 0, 0);
+        vb[e] = kImplicit ? 0 : (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rin_b, vo, 0, 0);
       }
     }
   };
   // the mappers' first two blocks of inputs need neither the table check nor
   // the tables: they are in flight while the tables are staged
   if (wid != 0 && nblk > 0) {
-    load_block(nblk - 1, ca, cb, cm);
-    if (nblk > 1) load_block(nblk - 2, na, nb, nm);
+    load_block(nblk - 1, ia[0], ib[0], im[0]);
+    load_block(nblk - 2, ia[1], ib[1], im[1]);
   }
   if (wid == 0) pc.mark_after_loads(1);  // table header and metadata are in
   const bool tab = tables_ok(th, a.M, a.tables_bytes, a.blob);  // uniform
@@ -1415,7 +1506,8 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
   if (!tab) status |= GAANS_ST_TABLES;
   if (tab) {
     if (kMode == kModeGaussian) stage_scales<kThreads>(scl, a.scale_table, a.n_scales, tid);
-    stage_tables<kThreads>(tb, lmeta, lent, nullptr, nullptr, bd, t_lo, t_hi, tid);
+    stage_tables<kThreads>(tb, lmeta, lent, nullptr, nullptr, bd, t_lo, t_hi, tid,
+                           ring_bytes + (uint32_t)G::kTail + 16u * (uint32_t)a.nt_cap);
     if (wid == 0) pc.mark(2);
     // the scale table's coarse level, after the staging barrier
     GaussCoarse gc{};
@@ -1423,11 +1515,11 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
 
     // this wave's steps per block: u = wid - 1 + kEncMappers e < SB
     const int nvalid = SB % kEncMappers == 0 ? kPer : (SB - wid + kEncMappers) / kEncMappers;
-    // the block's records into the LDS slot of block j, and its steps with
-    // escapes into the block's flag word
-    auto put_records = [&](int j, const uint4* r, bool fast, uint32_t esc_steps)
+    // the block's records into the LDS slot of the turn's parity b, and its
+    // steps with escapes into the slot's flag word
+    auto put_records = [&](int b, const uint4* r, bool fast, uint32_t esc_steps)
                            __attribute__((always_inline)) {
-      uint4* dst = recs + (j & 1) * SB * kLanes;
+      uint4* dst = recs + b * SB * kLanes;
       uint32_t eb = 0;
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
@@ -1438,19 +1530,19 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         else eb |= ballot((r[e].z & 256u) != 0u) != 0ull ? 1u << u : 0u;
       }
       if (eb != 0u && lane == 0)
-        __hip_atomic_fetch_or(&eflag[j & 1], eb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_or(&eflag[b], eb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
-    auto map_steps = [&](int j, auto lds_tag) __attribute__((always_inline)) {
+    auto map_steps = [&](int j, int b, auto lds_tag) __attribute__((always_inline)) {
       constexpr bool kLds = decltype(lds_tag)::value;
       uint4 r[kPer];
       enc_records<kMode, kImplicit, kLds, kPer>(a, tb, lane, j * SB + wid - 1, kEncMappers,
-                                                nvalid, len, start, ca, cb, cm, hash, status,
-                                                znib, r);
-      put_records(j, r, false, 0u);
+                                                nvalid, len, start, ia[b], ib[b], im[b], hash,
+                                                status, znib, r);
+      put_records(b, r, false, 0u);
     };
-    auto map_block = [&](int j) __attribute__((always_inline)) {
+    auto map_block = [&](int j, int b) __attribute__((always_inline)) {
       if (kMode == kModeGaussian)
-        gauss_indexes<kPer>(cb, scl, a.n_scales, a.scales_pow2, a.scale_bound, gc);
+        gauss_indexes<kPer>(ib[b], scl, a.n_scales, a.scales_pow2, a.scale_bound, gc);
       // A full block first tries the fast path, which checks by itself that
       // every table is staged and every value in range (and changes nothing
       // when it declines), so the check below runs only for the rest.
@@ -1458,9 +1550,9 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         uint4 r[kPer];
         uint32_t esc_steps = 0;
         if (enc_records_fast<kMode, kImplicit, kPer>(a, tb, lane, j * SB + wid - 1, kEncMappers,
-                                                     start, ca, cb, cm, hash, status, znib,
-                                                     esc_steps, r)) {
-          put_records(j, r, true, esc_steps);
+                                                     start, ia[b], ib[b], im[b], hash, status,
+                                                     znib, esc_steps, r)) {
+          put_records(b, r, true, esc_steps);
           return;
         }
       }
@@ -1472,12 +1564,12 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         for (int e = 0; e < kPer; ++e) {
           const int u = (wid - 1) + kEncMappers * e;
           outside |= u < SB && lane + kLanes * (j * SB + u) < len &&
-                     (uint32_t)(cb[e] - tb.t_lo) >= (uint32_t)tb.nt;
+                     (uint32_t)(ib[b][e] - tb.t_lo) >= (uint32_t)tb.nt;
         }
         lds = ballot(outside) == 0;
       }
-      if (lds) map_steps(j, std::true_type{});
-      else map_steps(j, std::false_type{});
+      if (lds) map_steps(j, b, std::true_type{});
+      else map_steps(j, b, std::false_type{});
     };
 
     // The coder and the mappers run separate code (the wave role is uniform
@@ -1490,51 +1582,55 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       // workgroup on the CU compete for the same SIMD.
       __builtin_amdgcn_s_setprio(3);
       const uint32_t spare = ring_mask + 1u + (uint32_t)lane;
+      constexpr bool kScalar = NM != 8;
+      uint32_t n = (uint32_t)-wp;
       __syncthreads();
       pc.mark(3);
       pc.cycles(12);
-      for (int j = nblk - 1; j >= 0; --j) {
+      for (int i = 0; i < nblk; ++i) {
         // coder: steps of block j, last to first
+        const int j = nblk - 1 - i, b = i & 1;
         if (fl - wp > (int)ring_mask + 1 - SB * kLanes) {
           ring_flush(wbuf, ring, wp, fl, lane, ring_mask);
           fl = wp;
         }
-        const uint4* src = recs + (j & 1) * SB * kLanes;
         // steps of the block with escapes when the coder lists them; cleared
         // for block j - 2
-        const uint32_t any_esc = kMList ? 0u : (uint32_t)uni((int)eflag[j & 1]);
-        if (!kMList && lane == 0) eflag[j & 1] = 0u;
-        const bool full = (j + 1) * SB <= T;
-        // the block's records in groups of at most 8 steps, last group first
-        constexpr int H = SB > 8 ? 8 : SB;
+        const uint32_t any_esc = kMList ? 0u : (uint32_t)uni((int)eflag[b]);
+        if (!kMList) eflag[b] = 0u;  // every lane: no exec-mask branch
+        const uint32_t rec = ring_bytes + 16u * (uint32_t)(b * SB * kLanes + lane);
+        if ((j + 1) * SB <= T) {
+          uint32_t kz[SB], kw[SB];
+          enc_steps<SB, kScalar, !kMList>(rec, spare, ring_mask, x, n, wp, kz, kw);
+          // escapes of the block (their bins are coded above): list them, last
+          // step first, so the list stays in position order
+          if (!kMList && __builtin_expect(any_esc != 0, 0)) {
 #pragma unroll
-        for (int h = SB / H - 1; h >= 0; --h) {
-          uint4 r[H];
-#pragma unroll
-          for (int k = 0; k < H; ++k) r[k] = src[(h * H + k) * kLanes + lane];
-          if (full) {
-            // common case: a full block, no per-step branches
-#pragma unroll
-            for (int k = H - 1; k >= 0; --k) {
-              emit_words(r[k].z, x, ring, wp, spare, ring_mask);
-              x = enc_apply(x, r[k]);
-            }
-          } else {
-#pragma unroll
-            for (int k = H - 1; k >= 0; --k) {
-              if (j * SB + h * H + k >= T) continue;
-              emit_words(r[k].z, x, ring, wp, spare, ring_mask);
-              x = enc_apply(x, r[k]);
+            for (int k = SB - 1; k >= 0; --k)
+              if (any_esc & (1u << k)) enc_escapes(kz[k], kw[k], esc_list, n_esc, lane);
+          }
+        } else {  // the unit's last steps, four and one at a time
+          int u = T - j * SB;
+          while (u > 0) {
+            if (u >= 4) {
+              u -= 4;
+              enc_steps<4, kScalar, false>(rec + 16u * (uint32_t)(u * kLanes), spare, ring_mask, x,
+                                           n, wp, nullptr, nullptr);
+            } else {
+              --u;
+              enc_steps<1, kScalar, false>(rec + 16u * (uint32_t)(u * kLanes), spare, ring_mask, x,
+                                           n, wp, nullptr, nullptr);
             }
           }
-          // escapes of the group (their bins are coded above): list them,
-          // last step first, so the list stays in position order
-          if (__builtin_expect(any_esc != 0, 0)) {
-#pragma unroll
-            for (int k = H - 1; k >= 0; --k)
-              if (any_esc & (1u << (h * H + k))) enc_escapes(r[k].z, r[k].w, esc_list, n_esc, lane);
+          const uint4* src = recs + b * SB * kLanes;
+          for (uint32_t left = any_esc; left != 0u;) {
+            const int k = 31 - __clz((int)left);
+            left &= ~(1u << k);
+            const uint4 rr = src[k * kLanes + lane];
+            enc_escapes(rr.z, rr.w, esc_list, n_esc, lane);
           }
         }
+        wp = kScalar ? uni(wp) : -uni((int)n);
         pc.bar_in();
         __syncthreads();
         pc.bar_out();
@@ -1542,9 +1638,13 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       pc.cycles(13);
       pc.mark(4);
     } else {
-      if (nblk > 0) map_block(nblk - 1);
+      if (nblk > 0) map_block(nblk - 1, 0);
+      load_block(nblk - 3, ia[0], ib[0], im[0]);
       __syncthreads();
-      for (int j = nblk - 1; j >= 0; --j) {
+      // While the coder codes block j (turn i): map block j - 1 (parity b) and
+      // load block j - 3.
+      auto turn = [&](int i, int b) __attribute__((always_inline)) {
+        const int j = nblk - 1 - i;
         // kMList: the first mapper wave lists the escapes of block j (their
         // bins are coded by the coder meanwhile) from the block's records,
         // last step first, so the list stays in position order, eight steps'
@@ -1552,10 +1652,10 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         // flags are cleared for block j - 2, which is mapped after the next
         // barrier.
         if (kMList && wid == 1) {
-          const uint32_t any_esc = (uint32_t)uni((int)eflag[j & 1]);
-          eflag[j & 1] = 0u;
+          const uint32_t any_esc = (uint32_t)uni((int)eflag[1 - b]);
+          eflag[1 - b] = 0u;
           if (any_esc != 0u) {
-            const uint4* src = recs + (j & 1) * SB * kLanes;
+            const uint4* src = recs + (1 - b) * SB * kLanes;
             constexpr int G8 = SB > 8 ? 8 : SB;
 #pragma unroll
             for (int hh = SB / G8 - 1; hh >= 0; --hh) {
@@ -1574,17 +1674,14 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
             }
           }
         }
-        if (j > 0) {  // mappers: block j - 1 while the coder codes block j
-#pragma unroll
-          for (int e = 0; e < kPer; ++e) {
-            ca[e] = na[e];
-            cb[e] = nb[e];
-            cm[e] = nm[e];
-          }
-          if (j > 1) load_block(j - 2, na, nb, nm);
-          map_block(j - 1);
-        }
+        if (j > 0) map_block(j - 1, b);
+        load_block(j - 3, ia[b], ib[b], im[b]);
         __syncthreads();
+      };
+      for (int i = 0; i < nblk; i += 2) {
+        turn(i, 1);
+        if (i + 1 >= nblk) break;
+        turn(i + 1, 0);
       }
     }
   }
@@ -3841,15 +3938,17 @@ EncKernel enc_kernel_sb(int sb, int nm) {
   return sb == 4 ? enc_kernel_nm<kMode, kImp, 4>(nm) : enc_kernel_nm<kMode, kImp, 8>(nm);
 }
 
-// Encode kernel of a mode, index kind, block size and mapper count; 16-step
-// blocks are built for explicit or computed indexes only (with table =
-// channel the 16-step kernel needs private scratch).
+// Encode kernel of a mode, index kind, block size and mapper count.
 EncKernel enc_kernel(int mode, bool imp, int sb, int nm) {
   if (sb == 16) {
     switch (mode) {
       case kModeGaussian: return enc_kernel_nm<kModeGaussian, false, 16>(nm);
-      case kModeLatents: return enc_kernel_nm<kModeLatents, false, 16>(nm);
-      default: return enc_kernel_nm<kModeSymbols, false, 16>(nm);
+      case kModeLatents:
+        return imp ? enc_kernel_nm<kModeLatents, true, 16>(nm)
+                   : enc_kernel_nm<kModeLatents, false, 16>(nm);
+      default:
+        return imp ? enc_kernel_nm<kModeSymbols, true, 16>(nm)
+                   : enc_kernel_nm<kModeSymbols, false, 16>(nm);
     }
   }
   switch (mode) {
@@ -3939,10 +4038,10 @@ int encode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
       mode == kModeGaussian ? align_up(4 * ((int64_t)n_scales + kGaussPad), 16) + 16 : 0;
   // 16-step blocks for long units only (the coder waits for the first
   // block to be mapped, so short units lose more than the per-block saving
-  // gains: measured slower at 96 steps, faster at 4,080), and with explicit
-  // or computed indexes only (with table = channel the 16-step kernel needs
-  // private scratch)
-  const bool long_units = L.seg_cap >= 512 * kLanes;
+  // gains: slower at 96 steps; at 384 steps 1x192x32x48, P = 16, 38.9 -> 33.8
+  // us and the batch-64 skew draw 49.8 -> 44.5 us; at 1,020 steps the
+  // 2160x3840 latent 94 -> 80 us)
+  const bool long_units = L.seg_cap >= 256 * kLanes;
   const bool gauss = mode == kModeGaussian;
   if (gauss) implicit = false;
   // The Gaussian mode's mappers (a scale-table search and table reads from
@@ -3951,7 +4050,7 @@ int encode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
   // (mean-scale hyperprior y, P = 4 and 16), and 16-step blocks give each
   // mapper wave two steps per block to overlap.
   const EncPlan plan = plan_encode(tables, L.P, L.U, dl, extra, !gauss,
-                                   (long_units || gauss) && !implicit);
+                                   long_units || gauss);
   const Stage& st = plan.st;
   size_t lds = plan.lds + (size_t)extra;
   if (lds > (size_t)dl.per_block)
