@@ -604,6 +604,7 @@ struct EncArgs {
   // numbered by the workgroup's slot on the CU
   uint32_t elect;
   PhaseBuf phase;
+  float* __restrict__ y_hat;  // latents: dequantized latents out [B, N], or NULL
 };
 
 // Encoder LDS layout (bytes): the output ring of `ring` u16 words (a power
@@ -733,8 +734,8 @@ template <int kMode, bool kImplicit, bool kLds, int KP>
 __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, int lane, int t0,
                                             int tstep, int nvalid, int len, int32_t start,
                                             const int32_t* in_a, const int32_t* in_b,
-                                            const float* in_m, uint32_t& hash, uint32_t& status,
-                                            uint32_t& znib, uint4* rec) {
+                                            const float* in_m, float* yh, uint32_t& hash,
+                                            uint32_t& status, uint32_t& znib, uint4* rec) {
   bool ok[KP];
   int32_t sym[KP], offset[KP];
   uint32_t ebase[KP], nsym[KP];
@@ -754,6 +755,8 @@ __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, in
       const bool rng = !(fabsf(r) < 2147483648.0f);
       status |= (ok[e] & rng) ? GAANS_ST_RANGE : 0u;
       sym[e] = (int32_t)(rng ? 0.0f : r);
+      if (kMode == kModeLatents && yh && act)
+        yh[unit_pos(0, a.S, p)] = __fadd_rn((float)sym[e], in_m[e]);
     } else {
       sym[e] = in_a[e];
     }
@@ -826,7 +829,7 @@ template <int kMode, bool kImplicit, int KP>
 __device__ __forceinline__ bool enc_records_fast(const EncArgs& a, const Tabs& tb, int lane,
                                                  int t0, int tstep, int32_t start,
                                                  const int32_t* in_a, const int32_t* in_b,
-                                                 const float* in_m, uint32_t& hash,
+                                                 const float* in_m, float* yh, uint32_t& hash,
                                                  uint32_t& status, uint32_t& znib,
                                                  uint32_t& esc_steps, uint4* rec) {
   int32_t sym[KP];
@@ -845,6 +848,8 @@ __device__ __forceinline__ bool enc_records_fast(const EncArgs& a, const Tabs& t
       const float r = rintf(__fsub_rn(__int_as_float(in_a[e]), in_m[e]));
       bad |= ballot(!(fabsf(r) < 2147483648.0f));
       sym[e] = (int32_t)r;
+      if (kMode == kModeLatents && yh)
+        yh[unit_pos(0, a.S, p)] = __fadd_rn((float)sym[e], in_m[e]);
     } else {
       sym[e] = in_a[e];
     }
@@ -1513,6 +1518,8 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
     GaussCoarse gc{};
     if (kMode == kModeGaussian && wid != 0) gc = gauss_coarse(scl, a.n_scales);
 
+    // the unit's part of the dequantized latents, when the caller wants them
+    float* yh = kMode == kModeLatents && a.y_hat ? a.y_hat + row + start : nullptr;
     // this wave's steps per block: u = wid - 1 + kEncMappers e < SB
     const int nvalid = SB % kEncMappers == 0 ? kPer : (SB - wid + kEncMappers) / kEncMappers;
     // the block's records into the LDS slot of the turn's parity b, and its
@@ -1536,8 +1543,8 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       constexpr bool kLds = decltype(lds_tag)::value;
       uint4 r[kPer];
       enc_records<kMode, kImplicit, kLds, kPer>(a, tb, lane, j * SB + wid - 1, kEncMappers,
-                                                nvalid, len, start, ia[b], ib[b], im[b], hash,
-                                                status, znib, r);
+                                                nvalid, len, start, ia[b], ib[b], im[b], yh,
+                                                hash, status, znib, r);
       put_records(b, r, false, 0u);
     };
     auto map_block = [&](int j, int b) __attribute__((always_inline)) {
@@ -1550,7 +1557,7 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         uint4 r[kPer];
         uint32_t esc_steps = 0;
         if (enc_records_fast<kMode, kImplicit, kPer>(a, tb, lane, j * SB + wid - 1, kEncMappers,
-                                                     start, ia[b], ib[b], im[b], hash, status,
+                                                     start, ia[b], ib[b], im[b], yh, hash, status,
                                                      znib, esc_steps, r)) {
           put_records(b, r, true, esc_steps);
           return;
@@ -4149,6 +4156,7 @@ void encode_bind(int mode, EncArgs& a, const Layout& L, const int32_t* symbols, 
   a.ctrl = static_cast<uint32_t*>(ctrl);
   a.info_out = info_out;
   a.look = reinterpret_cast<uint64_t*>(w + L.o_look);
+  a.y_hat = nullptr;
   a.out = nullptr;  // stage 1 only unless the caller fuses the pack (encode_fuse)
   a.out_bytes = 0;
   a.phase = g_phase;
@@ -4708,22 +4716,10 @@ int gaans_plan_decode(const gaans_tables* tables, int32_t mode, int32_t explicit
   return GAANS_OK;
 }
 
-int gaans_run_encode(const gaans_plan* plan, void* stream, const void* in0, const void* in1,
-                     const void* in2, const void* in3, void* workspace_dev,
-                     int64_t workspace_bytes, void* ctrl_dev, uint8_t* out_dev,
-                     int64_t out_bytes, uint64_t* info_host) {
-  if (!info_host) return fail(GAANS_EINVAL, "info_host pointer is NULL");
-  uint32_t* done = reinterpret_cast<uint32_t*>(&info_host[2]);  // low half of info[2]
-  __atomic_store_n(done, 0u, __ATOMIC_RELEASE);
-  const int rc = gaans_enqueue_encode(plan, stream, in0, in1, in2, in3, workspace_dev,
-                                      workspace_bytes, ctrl_dev, out_dev, out_bytes, info_host);
-  return rc ? rc : wait_word(stream, done);
-}
-
-int gaans_enqueue_encode(const gaans_plan* plan, void* stream, const void* in0, const void* in1,
-                         const void* in2, const void* in3, void* workspace_dev,
-                         int64_t workspace_bytes, void* ctrl_dev, uint8_t* out_dev,
-                         int64_t out_bytes, uint64_t* info_out) {
+static int enqueue_encode(const gaans_plan* plan, void* stream, const void* in0, const void* in1,
+                          const void* in2, const void* in3, float* y_hat, void* workspace_dev,
+                          int64_t workspace_bytes, void* ctrl_dev, uint8_t* out_dev,
+                          int64_t out_bytes, uint64_t* info_out) {
   const EncPlanRec* r = reinterpret_cast<const EncPlanRec*>(plan);
   if (!r || r->h.magic != kPlanEncMagic)
     return fail(GAANS_EINVAL, "not an encode plan (gaans_plan_encode)");
@@ -4751,8 +4747,40 @@ int gaans_enqueue_encode(const gaans_plan* plan, void* stream, const void* in0, 
   if (rc || (rc = plan_device(r->h))) return rc;
   EncLaunch e = r->e;
   encode_bind(mode, e.a, L, symbols, y, medians, indexes, &g, workspace_dev, ctrl_dev, info_out);
+  e.a.y_hat = y_hat;
   if ((rc = encode_fuse(e.a, L, out_dev, out_bytes))) return rc;
   return encode_launch(e, stream);
+}
+
+int gaans_run_encode(const gaans_plan* plan, void* stream, const void* in0, const void* in1,
+                     const void* in2, const void* in3, void* workspace_dev,
+                     int64_t workspace_bytes, void* ctrl_dev, uint8_t* out_dev,
+                     int64_t out_bytes, uint64_t* info_host) {
+  if (!info_host) return fail(GAANS_EINVAL, "info_host pointer is NULL");
+  uint32_t* done = reinterpret_cast<uint32_t*>(&info_host[2]);  // low half of info[2]
+  __atomic_store_n(done, 0u, __ATOMIC_RELEASE);
+  const int rc = gaans_enqueue_encode(plan, stream, in0, in1, in2, in3, workspace_dev,
+                                      workspace_bytes, ctrl_dev, out_dev, out_bytes, info_host);
+  return rc ? rc : wait_word(stream, done);
+}
+
+int gaans_enqueue_encode(const gaans_plan* plan, void* stream, const void* in0, const void* in1,
+                         const void* in2, const void* in3, void* workspace_dev,
+                         int64_t workspace_bytes, void* ctrl_dev, uint8_t* out_dev,
+                         int64_t out_bytes, uint64_t* info_out) {
+  return enqueue_encode(plan, stream, in0, in1, in2, in3, nullptr, workspace_dev,
+                        workspace_bytes, ctrl_dev, out_dev, out_bytes, info_out);
+}
+
+int gaans_enqueue_encode_latents(const gaans_plan* plan, void* stream, const float* y,
+                                 const float* medians, const int32_t* indexes, float* y_hat,
+                                 void* workspace_dev, int64_t workspace_bytes, void* ctrl_dev,
+                                 uint8_t* out_dev, int64_t out_bytes, uint64_t* info_out) {
+  const EncPlanRec* r = reinterpret_cast<const EncPlanRec*>(plan);
+  if (r && r->h.magic == kPlanEncMagic && r->h.mode != GAANS_MODE_LATENTS)
+    return fail(GAANS_EINVAL, "not a plan of GAANS_MODE_LATENTS");
+  return enqueue_encode(plan, stream, y, medians, indexes, nullptr, y_hat, workspace_dev,
+                        workspace_bytes, ctrl_dev, out_dev, out_bytes, info_out);
 }
 
 int gaans_run_decode(const gaans_plan* plan, void* stream, const uint8_t* payload_dev,

@@ -154,6 +154,8 @@ def _declare(L) -> None:
         "gaans_run_encode": ([p, p, p, p, p, p, p, i64, p, p, i64, p], ctypes.c_int),
         "gaans_run_decode": ([p, p, p, i64, p, p, p, p, p, p], ctypes.c_int),
         "gaans_enqueue_encode": ([p, p, p, p, p, p, p, i64, p, p, i64, p], ctypes.c_int),
+        "gaans_enqueue_encode_latents": ([p, p, p, p, p, p, p, i64, p, p, i64, p],
+                                         ctypes.c_int),
         "gaans_enqueue_decode": ([p, p, p, i64, p, p, p, p, p, p], ctypes.c_int),
         # struct addresses (c_void_p): one argument to convert per call
         "gaans_run_encode_call": ([p], ctypes.c_int),

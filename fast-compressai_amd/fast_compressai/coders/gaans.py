@@ -36,6 +36,7 @@ from .errors import CoderInputError
 from .tables import PreparedTables
 
 CLONE_SLACK_BYTES = 32 << 20  # keep a view of the worst-case buffer below this waste
+MAX_SLOTS = 8  # pinned word sets kept per stream (32 bytes each)
 
 
 class _StreamState:
@@ -53,6 +54,20 @@ class _StreamState:
         self.workspace = torch.zeros(0, dtype=torch.uint8, device=device)
         self.device = device
         self.lock = threading.Lock()
+        self.slots: list = []  # pinned words of calls in flight, returned when they end
+
+    def slot(self) -> torch.Tensor:
+        """Pinned completion words for a call that is waited for later (the
+        caller holds ``lock``; ``give_back`` afterwards)."""
+        slot = self.slots.pop() if self.slots else torch.empty(4, dtype=torch.int64,
+                                                               pin_memory=True)
+        slot.zero_()
+        return slot
+
+    def give_back(self, slot: torch.Tensor) -> None:
+        with self.lock:
+            if len(self.slots) < MAX_SLOTS:
+                self.slots.append(slot)
 
     def ws(self, nbytes: int) -> torch.Tensor:
         """The workspace, grown (and zeroed) when a shape needs more; the
@@ -259,6 +274,10 @@ def _run_encode(tables: PreparedTables, mode: int, explicit: bool, B: int, N: in
     when the buffer would waste more than CLONE_SLACK_BYTES)."""
     out, total, lay = _run_encode_raw(tables, mode, explicit, B, N, C, P, S, device, in0, in1,
                                       in2, in3, what, n_scales, bound)
+    return _chunks(out, total, lay, S, B)
+
+
+def _chunks(out: torch.Tensor, total: int, lay, S: int, B: int) -> EncodedChunks:
     packed = out[:total]
     if lay.max_payload_bytes - total > CLONE_SLACK_BYTES:
         packed = packed.clone()
@@ -433,6 +452,92 @@ def decode(packed: torch.Tensor, tables: PreparedTables, B: int, N: int, C: int,
                            torch.float32, "GA-ANS decode")
     return _run_decode(tables, _native.MODE_SYMBOLS, indexes is not None, B, N, C, P, segments,
                        device, packed, _ptr(indexes), None, None, torch.int32, "GA-ANS decode")
+
+
+class _Pending:
+    """A call enqueued on the current stream whose completion word is still to
+    come.  ``finish`` waits for it and must be called once, whatever else
+    happens in between: the word's memory is the call's until then."""
+
+    def __init__(self, st: _StreamState, stream_ptr: int, slot: torch.Tensor, word: int,
+                 result) -> None:
+        self._st, self._sp, self._slot, self._word, self._result = st, stream_ptr, slot, word, result
+
+    def finish(self):
+        _native.check(_native.lib().gaans_wait_host_word(
+            self._sp, self._slot.data_ptr() + self._word), "GA-ANS wait")
+        words = self._slot.tolist()
+        self._st.give_back(self._slot)
+        return self._result(words)
+
+
+def encode_latents_begin(tables: PreparedTables, B: int, N: int, C: int, P: int, device, *,
+                         y: torch.Tensor, medians: torch.Tensor, y_hat: torch.Tensor | None,
+                         segments: int = 1) -> _Pending:
+    """``encode`` of latents (channel-major tables) without the wait: work that
+    needs only ``y_hat`` (fp32 [B, N], written by the same kernel) is enqueued
+    behind it, and the host prepares that work while the GPU codes.
+    ``finish()`` returns the ``EncodedChunks``."""
+    index = _index(device)
+    prev = _enter_device(index)
+    try:
+        _, plan, lay = _plan(tables, False, _native.MODE_LATENTS, False, B, N, C, P, segments,
+                             index)
+        sp = torch._C._cuda_getCurrentRawStream(index)
+        st = _state(index, sp)
+        out = torch.empty(lay.max_payload_bytes, dtype=torch.uint8, device=st.device)
+        with st.lock:
+            ws, slot = st.ws(lay.workspace_bytes), st.slot()
+            rc = _native.lib().gaans_enqueue_encode_latents(
+                plan, sp, y.data_ptr(), medians.data_ptr(), None, _ptr(y_hat), ws.data_ptr(),
+                ws.numel(), st.ctrl_ptr, out.data_ptr(), lay.max_payload_bytes, slot.data_ptr())
+        if rc:
+            _native.check(rc, "GA-ANS encode")
+    finally:
+        if prev is not None:
+            torch.cuda.set_device(prev)
+
+    def result(words):
+        word = words[2]  # 1 | status << 1 | payload bytes << 16
+        if (word >> 1) & 0x7FFF:
+            raise CoderInputError("GA-ANS encode failed: "
+                                  f"{_native.describe_status((word >> 1) & 0x7FFF)}")
+        return _chunks(out, word >> 16, lay, segments, B)
+
+    return _Pending(st, sp, slot, 16, result)
+
+
+def decode_latents_begin(packed: torch.Tensor, tables: PreparedTables, B: int, N: int, C: int,
+                         P: int, device, *, medians: torch.Tensor,
+                         segments: int = 1) -> tuple[_Pending, torch.Tensor]:
+    """``decode`` to fp32 latents (channel-major tables) without the wait:
+    returns the pending call and y_hat [B, N], which work enqueued behind it on
+    this stream may read.  y_hat is meaningful only if ``finish()`` returns."""
+    index = _index(device)
+    prev = _enter_device(index)
+    try:
+        _, plan, _lay = _plan(tables, True, _native.MODE_LATENTS, False, B, N, C, P, segments,
+                              index)
+        sp = torch._C._cuda_getCurrentRawStream(index)
+        st = _state(index, sp)
+        out = torch.empty((B, N), dtype=torch.float32, device=st.device)
+        with st.lock:
+            slot = st.slot()
+            rc = _native.lib().gaans_enqueue_decode(plan, sp, packed.data_ptr(), packed.numel(),
+                                                    medians.data_ptr(), None, None,
+                                                    out.data_ptr(), st.ctrl_ptr, slot.data_ptr())
+        if rc:
+            _native.check(rc, "GA-ANS decode")
+    finally:
+        if prev is not None:
+            torch.cuda.set_device(prev)
+
+    def result(words):
+        status = (words[0] >> 32) >> 1  # second 32-bit word: 1 | status << 1
+        if status:
+            raise CoderInputError(f"warp_div decode failed: {_native.describe_status(status)}")
+
+    return _Pending(st, sp, slot, 4, result), out
 
 
 def encode_gaussian(tables: PreparedTables, B: int, N: int, C: int, P: int, device, *,

@@ -414,6 +414,15 @@ int gaans_enqueue_encode(const gaans_plan* plan, void* stream, const void* in0, 
                          int64_t workspace_bytes, void* ctrl_dev, uint8_t* out_dev,
                          int64_t out_bytes, uint64_t* info_out);
 
+/* gaans_enqueue_encode of a GAANS_MODE_LATENTS plan that also writes the
+ * dequantized latents y_hat = fp32(symbol) + median (fp32 [B, N], or NULL for
+ * none) from the lanes that quantize them: the input of a hyperprior's h_s
+ * without another pass over the latents.  No counterpart in the reference. */
+int gaans_enqueue_encode_latents(const gaans_plan* plan, void* stream, const float* y,
+                                 const float* medians, const int32_t* indexes, float* y_hat,
+                                 void* workspace_dev, int64_t workspace_bytes, void* ctrl_dev,
+                                 uint8_t* out_dev, int64_t out_bytes, uint64_t* info_out);
+
 /* Decode with a plan into out_dev (int32 symbols for GAANS_MODE_SYMBOLS, fp32
  * y_hat otherwise, [B, N]) and wait for the completion word status_host[1]
  * (pinned host memory, 2 u32; cleared by the run); status_host[0] and the
