@@ -9,7 +9,7 @@
 // by the CPU oracle (oracle/gaans_oracle.c).
 //
 // Work mapping: one workgroup per coding unit (a coder wave and mapper
-// waves for encode; one more wave, the escape reader, for decode).  A chunk's
+// waves for encode; one more wave, the stream and escape reader, for decode).  A chunk's
 // S units run on S CUs, so S > 1 puts a launch of few long chunks on more of
 // the chip.
 //  - Wave 0 is the coder: it owns the 64 lane states and runs only the
@@ -28,8 +28,8 @@
 //    few) are staged in LDS by the whole workgroup; others are read through
 //    L1/L2.
 //  - encode: emitted words go to an LDS ring, flushed to a per-chunk staging
-//    slot when full; decode: the word stream is prefetched from HBM into
-//    registers and copied into an LDS ring ahead of use.
+//    slot when full; decode: the last wave prefetches the word stream from HBM
+//    into registers and copies it into an LDS ring ahead of use.
 //  - The last workgroup of a launch (device-scope counter in a caller-owned
 //    control block) scans the chunk sizes into payload offsets (encode) or
 //    reduces the status words (decode) and writes them to caller memory.
@@ -1539,17 +1539,34 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       if (eb != 0u && lane == 0)
         __hip_atomic_fetch_or(&eflag[b], eb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
+    int32_t ca[kPer], cb[kPer];  // the inputs of the block being mapped
+    float cm[kPer];
     auto map_steps = [&](int j, int b, auto lds_tag) __attribute__((always_inline)) {
       constexpr bool kLds = decltype(lds_tag)::value;
       uint4 r[kPer];
       enc_records<kMode, kImplicit, kLds, kPer>(a, tb, lane, j * SB + wid - 1, kEncMappers,
-                                                nvalid, len, start, ia[b], ib[b], im[b], yh,
-                                                hash, status, znib, r);
+                                                nvalid, len, start, ca, cb, cm, yh, hash, status,
+                                                znib, r);
       put_records(b, r, false, 0u);
     };
+    // Maps block j (register set b) and refills the set with block j - 2.  The
+    // loads go out before the mapping, two whole turns ahead of their use: with
+    // inputs that no L2 holds (three input sets in rotation) batch-64 uniform
+    // took 84.9 us per call with the loads after it.
     auto map_block = [&](int j, int b) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        ca[e] = ia[b][e];
+        cb[e] = ib[b][e];
+        cm[e] = im[b][e];
+        // the set's loads are waited for here, before the next ones are issued
+        asm volatile("" : "+v"(ca[e]));
+        if (!kImplicit) asm volatile("" : "+v"(cb[e]));
+        if (kMode != kModeSymbols) asm volatile("" : "+v"(cm[e]));
+      }
+      load_block(j - 2, ia[b], ib[b], im[b]);
       if (kMode == kModeGaussian)
-        gauss_indexes<kPer>(ib[b], scl, a.n_scales, a.scales_pow2, a.scale_bound, gc);
+        gauss_indexes<kPer>(cb, scl, a.n_scales, a.scales_pow2, a.scale_bound, gc);
       // A full block first tries the fast path, which checks by itself that
       // every table is staged and every value in range (and changes nothing
       // when it declines), so the check below runs only for the rest.
@@ -1557,8 +1574,8 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         uint4 r[kPer];
         uint32_t esc_steps = 0;
         if (enc_records_fast<kMode, kImplicit, kPer>(a, tb, lane, j * SB + wid - 1, kEncMappers,
-                                                     start, ia[b], ib[b], im[b], yh, hash, status,
-                                                     znib, esc_steps, r)) {
+                                                     start, ca, cb, cm, yh, hash, status, znib,
+                                                     esc_steps, r)) {
           put_records(b, r, true, esc_steps);
           return;
         }
@@ -1571,7 +1588,7 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         for (int e = 0; e < kPer; ++e) {
           const int u = (wid - 1) + kEncMappers * e;
           outside |= u < SB && lane + kLanes * (j * SB + u) < len &&
-                     (uint32_t)(ib[b][e] - tb.t_lo) >= (uint32_t)tb.nt;
+                     (uint32_t)(cb[e] - tb.t_lo) >= (uint32_t)tb.nt;
         }
         lds = ballot(outside) == 0;
       }
@@ -1646,10 +1663,8 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       pc.mark(4);
     } else {
       if (nblk > 0) map_block(nblk - 1, 0);
-      load_block(nblk - 3, ia[0], ib[0], im[0]);
       __syncthreads();
-      // While the coder codes block j (turn i): map block j - 1 (parity b) and
-      // load block j - 3.
+      // While the coder codes block j (turn i): map block j - 1 (parity b).
       auto turn = [&](int i, int b) __attribute__((always_inline)) {
         const int j = nblk - 1 - i;
         // kMList: the first mapper wave lists the escapes of block j (their
@@ -1682,7 +1697,6 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
           }
         }
         if (j > 0) map_block(j - 1, b);
-        load_block(j - 3, ia[b], ib[b], im[b]);
         __syncthreads();
       };
       for (int i = 0; i < nblk; i += 2) {
@@ -1841,7 +1855,7 @@ __global__ __launch_bounds__(256) void k_pack(PackArgs a) {
 // ============================================================================
 
 // Decode workgroup: wave 0 is the coder, waves 1..kMappers the mappers, the
-// last wave the escape reader.
+// last wave the stream and escape reader.
 constexpr int kDecWaves = kMappers + 2;
 constexpr int kDecThreads = kDecWaves * kLanes;
 constexpr int kEscWave = kDecWaves - 1;
@@ -2541,7 +2555,7 @@ __device__ __forceinline__ StepShadow step_shadow(uint64_t m, uint32_t hi, uint3
 // entry read.  Cycles per step on MI355X with one workgroup per CU (uniform
 // 255-symbol tables, no dense steps): 335 with the compiler's step and the
 // stream, escape masks and stores on this wave, 235 so.  512x768, P = 4: 23.1
-// -> 19.7 us; 2160x3840, P = 8: 224 -> 178 us.
+// -> 18.6 us; 2160x3840, P = 8: 224 -> 173 us.
 //
 // A step's state is a guess until the test for dense entries, after the next
 // step's entry read: a dense step is then looked up and its update, ring read
@@ -2660,7 +2674,7 @@ __device__ __forceinline__ uint32_t dec_block(const Tabs& tb, uint32_t rec, uint
 // with the compiler's 71 instructions and selects and 8-step blocks, 421 so (4
 // address operations, 5 from the entry to the starts' address, 19 from the
 // starts to the ring read, three LDS round trips; 16-step blocks fit beside
-// the tables since the records are 4 bytes).  P = 16: 94.7 -> 76.9 us, P = 4:
+// the tables since the records are 4 bytes).  P = 16: 94.7 -> 74.3 us, P = 4:
 // 29.9 -> 26.2 us.
 template <int SB, int NS, uint32_t kLutOff>
 __device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, uint32_t rn,
