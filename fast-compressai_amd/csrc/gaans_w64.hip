@@ -1549,22 +1549,26 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
                                                 znib, r);
       put_records(b, r, false, 0u);
     };
-    // Maps block j (register set b) and refills the set with block j - 2.  The
-    // loads go out before the mapping, two whole turns ahead of their use: with
-    // inputs that no L2 holds (three input sets in rotation) batch-64 uniform
-    // took 84.9 us per call with the loads after it.
-    auto map_block = [&](int j, int b) __attribute__((always_inline)) {
+    // Takes block j out of register set b and refills the set with block j - 2:
+    // the loads go out before block j is mapped, two whole turns ahead of their
+    // use.  Every turn does this, also the one that maps nothing (its loads lie
+    // outside the unit and read 0): where the loads are conditional, the wait for
+    // one set becomes a wait for both.
+    auto take_block = [&](int j, int b) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
-        ca[e] = ia[b][e];
-        cb[e] = ib[b][e];
-        cm[e] = im[b][e];
+        // a copy that the register allocator keeps (it would put the new loads
+        // elsewhere and copy them back at the end of the turn, waiting for them);
         // the set's loads are waited for here, before the next ones are issued
-        asm volatile("" : "+v"(ca[e]));
-        if (!kImplicit) asm volatile("" : "+v"(cb[e]));
-        if (kMode != kModeSymbols) asm volatile("" : "+v"(cm[e]));
+        cb[e] = 0;
+        cm[e] = 0.0f;
+        asm volatile("v_mov_b32 %0, %1" : "=v"(ca[e]) : "v"(ia[b][e]));
+        if (!kImplicit) asm volatile("v_mov_b32 %0, %1" : "=v"(cb[e]) : "v"(ib[b][e]));
+        if (kMode != kModeSymbols) asm volatile("v_mov_b32 %0, %1" : "=v"(cm[e]) : "v"(im[b][e]));
       }
       load_block(j - 2, ia[b], ib[b], im[b]);
+    };
+    auto map_block = [&](int j, int b) __attribute__((always_inline)) {
       if (kMode == kModeGaussian)
         gauss_indexes<kPer>(cb, scl, a.n_scales, a.scales_pow2, a.scale_bound, gc);
       // A full block first tries the fast path, which checks by itself that
@@ -1662,6 +1666,7 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       pc.cycles(13);
       pc.mark(4);
     } else {
+      take_block(nblk - 1, 0);
       if (nblk > 0) map_block(nblk - 1, 0);
       __syncthreads();
       // While the coder codes block j (turn i): map block j - 1 (parity b).
@@ -1696,6 +1701,7 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
             }
           }
         }
+        take_block(j - 1, b);
         if (j > 0) map_block(j - 1, b);
         __syncthreads();
       };
