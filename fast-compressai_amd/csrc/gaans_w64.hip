@@ -1678,7 +1678,7 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         // escape words read at a time (one wait for each group).  The steps'
         // flags are cleared for block j - 2, which is mapped after the next
         // barrier.
-        if (kMList && wid == 1) {
+        if (kMList && wid == 1 && j >= 0) {
           const uint32_t any_esc = (uint32_t)uni((int)eflag[1 - b]);
           eflag[1 - b] = 0u;
           if (any_esc != 0u) {
@@ -1703,11 +1703,13 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         }
         take_block(j - 1, b);
         if (j > 0) map_block(j - 1, b);
-        __syncthreads();
+        if (j >= 0) __syncthreads();  // as many as the coder's blocks
       };
+      // Two turns each time round, the second one empty past the last block: a
+      // way out between them would be one more path to the first turn's wait,
+      // on which the set it waits for is the last one loaded.
       for (int i = 0; i < nblk; i += 2) {
         turn(i, 1);
-        if (i + 1 >= nblk) break;
         turn(i + 1, 0);
       }
     }
