@@ -58,10 +58,12 @@ class _StreamState:
 
     def slot(self) -> torch.Tensor:
         """Pinned completion words for a call that is waited for later (the
-        caller holds ``lock``; ``give_back`` afterwards)."""
+        caller holds ``lock``; ``give_back`` afterwards).  Cleared through the
+        host view: words made under ``torch.inference_mode`` refuse torch's own
+        in-place operations once it has ended."""
         slot = self.slots.pop() if self.slots else torch.empty(4, dtype=torch.int64,
                                                                pin_memory=True)
-        slot.zero_()
+        slot.numpy()[:] = 0
         return slot
 
     def give_back(self, slot: torch.Tensor) -> None:

@@ -82,3 +82,18 @@ def test_error_of_z_is_raised_first(gpu_device, h_s_fails):
     again = fast.compress(x)["strings"]
     assert [p.to_bytes() for p in again] == [p.to_bytes() for p in out["strings"]]
     assert torch.equal(fast.decompress(out["strings"], out["shape"])["x_hat"], good)
+
+
+def test_calls_in_and_out_of_inference_mode(gpu_device):
+    model = make_hyperprior(mean_scale=True).to(gpu_device)
+    codec = fast_compressai.accelerate(model, P=4, device=str(gpu_device))._coder
+    x = torch.rand(1, 3, 64, 64, device=gpu_device)
+    # the first call makes this stream's words
+    gaans._state(0, torch.cuda.current_stream(gpu_device).cuda_stream).slots.clear()
+    got = []
+    for mode in (True, False, True):
+        with torch.inference_mode(mode), torch.no_grad():
+            out = codec.encode_latents(codec.analyze(x))
+            y_hat = codec.decode_latents(out["strings"], out["shape"])
+            got.append([p.to_bytes() for p in out["strings"]] + [y_hat.cpu().numpy().tobytes()])
+    assert got[0] == got[1] == got[2]
