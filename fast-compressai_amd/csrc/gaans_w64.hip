@@ -1354,6 +1354,17 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
   // workgroups per CU the mappers have no time to spare (batch-64 uniform 67
   // -> 72 us with the listing moved).
   constexpr bool kMList = NM == 8;
+  // How far ahead the mappers load a block's inputs.  Two turns before the block
+  // is mapped, into two register sets, with a CU to each workgroup (hyperprior
+  // y, P = 16: kernel 43.8 -> 42.0 us) and with 16-step blocks, which long units
+  // have (64 x 192 x 32 x 48 latents, P = 16: 87.8 us a call with one turn, 85.0
+  // with two).  One turn, into one set, with 8- and 4-step blocks and four
+  // mappers: the CU's other workgroups cover the wait, and no turn is spent
+  // loading outside the unit (batch-64 uniform, three input sets in rotation:
+  // 83.8 us a call with two turns, 81.5 with one; 35 x 192 x 124 x 6 latents, P =
+  // 4, units of 47 steps: 82.4 and 80.8).
+  constexpr bool kTwoAhead = NM == 8 || SB == 16;
+  static_assert(kTwoAhead || !kMList, "the one-turn loop lists no escapes");
   extern __shared__ __align__(16) uint8_t smem[];
   uint16_t* ring = reinterpret_cast<uint16_t*>(smem);
   const uint32_t ring_mask = a.ring_mask;  // ring words - 1
@@ -1449,12 +1460,13 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
   tb.lsub = nullptr;
   // mapper wave w (1..kEncMappers) owns steps u = w - 1 + kEncMappers e of every block
   // (steps a wave does not own keep these zeros)
-  // Inputs of two blocks, by the parity of the block's turn (block nblk - 1 is
-  // turn 0): two sets and a loop unrolled twice, not copies from one to the
-  // other, which would wait for the loads that were just issued.  A block
-  // before the first loads nothing (its offsets are out of range), so the loads
-  // need no condition: after one, the compiler waits for every outstanding load
-  // instead of counting.
+  // Inputs of two blocks (see the mappers' loop).  kTwoAhead: by the parity of
+  // the block's turn (block nblk - 1 is turn 0): two sets and a loop unrolled
+  // twice, not copies from one to the other, which would wait for the loads that
+  // were just issued.  A block before the first loads nothing (its offsets are
+  // out of range), so the loads need no condition: after one, the compiler waits
+  // for every outstanding load instead of counting.  Without kTwoAhead: the next
+  // block's, [0] for the first block only and [1] from then on.
   int32_t ia[2][kPer] = {}, ib[2][kPer] = {};
   float im[2][kPer] = {};
   // The unit's inputs as buffer resources over its len positions: a load's
@@ -1568,6 +1580,15 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       }
       load_block(j - 2, ia[b], ib[b], im[b]);
     };
+    // Without kTwoAhead: set b becomes the block being mapped.
+    auto take_next = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        ca[e] = ia[b][e];
+        cb[e] = ib[b][e];
+        cm[e] = im[b][e];
+      }
+    };
     auto map_block = [&](int j, int b) __attribute__((always_inline)) {
       if (kMode == kModeGaussian)
         gauss_indexes<kPer>(cb, scl, a.n_scales, a.scales_pow2, a.scale_bound, gc);
@@ -1666,9 +1687,6 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
       pc.cycles(13);
       pc.mark(4);
     } else {
-      take_block(nblk - 1, 0);
-      if (nblk > 0) map_block(nblk - 1, 0);
-      __syncthreads();
       // While the coder codes block j (turn i): map block j - 1 (parity b).
       auto turn = [&](int i, int b) __attribute__((always_inline)) {
         const int j = nblk - 1 - i;
@@ -1705,12 +1723,30 @@ __global__ __launch_bounds__((NM + 1) * kLanes) void k_encode(EncArgs a) {
         if (j > 0) map_block(j - 1, b);
         if (j >= 0) __syncthreads();  // as many as the coder's blocks
       };
-      // Two turns each time round, the second one empty past the last block: a
-      // way out between them would be one more path to the first turn's wait,
-      // on which the set it waits for is the last one loaded.
-      for (int i = 0; i < nblk; i += 2) {
-        turn(i, 1);
-        turn(i + 1, 0);
+      if constexpr (kTwoAhead) {
+        take_block(nblk - 1, 0);
+        if (nblk > 0) map_block(nblk - 1, 0);
+        __syncthreads();
+        // Two turns each time round, the second one empty past the last block: a
+        // way out between them would be one more path to the first turn's wait,
+        // on which the set it waits for is the last one loaded.
+        for (int i = 0; i < nblk; i += 2) {
+          turn(i, 1);
+          turn(i + 1, 0);
+        }
+      } else {
+        take_next(0);
+        if (nblk > 0) map_block(nblk - 1, 0);
+        __syncthreads();
+        for (int i = 0; i < nblk; ++i) {
+          const int j = nblk - 1 - i;
+          if (j > 0) {
+            take_next(1);
+            if (j > 1) load_block(j - 2, ia[1], ib[1], im[1]);
+            map_block(j - 1, (i + 1) & 1);
+          }
+          __syncthreads();
+        }
       }
     }
   }
