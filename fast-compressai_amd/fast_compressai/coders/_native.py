@@ -15,7 +15,7 @@ import threading
 from .errors import CoderDependencyError
 
 LIB_NAME = "libgaans_w64.so"
-ABI_VERSION = 14
+ABI_VERSION = 15
 CTRL_BYTES = 256
 PLAN_BYTES = 1536  # GAANS_PLAN_BYTES
 PHASE_SLOTS = 16  # GAANS_PHASE_SLOTS
@@ -181,11 +181,12 @@ def lib():
                     f"GA-ANS HIP library is not built ({path}); run __graft_entry__.build()")
             try:
                 L = ctypes.CDLL(path)
+                # before the declarations, which an older library lacks some of
+                if L.gaans_abi_version() != ABI_VERSION:
+                    raise CoderDependencyError("GA-ANS HIP library ABI version mismatch")
                 _declare(L)
             except (OSError, AttributeError) as exc:
                 raise CoderDependencyError(f"GA-ANS HIP library could not be loaded: {exc}") from exc
-            if L.gaans_abi_version() != ABI_VERSION:
-                raise CoderDependencyError("GA-ANS HIP library ABI version mismatch")
             _lib = L
     return _lib
 

@@ -62,7 +62,7 @@
 extern "C" {
 #endif
 
-#define GAANS_ABI_VERSION 14
+#define GAANS_ABI_VERSION 15
 #define GAANS_CTRL_BYTES 256
 
 /* return codes */

@@ -4,9 +4,11 @@ tables whose digest and decode lookup agree with the oracle / a brute-force
 search.  No kernel is launched here."""
 
 import ctypes
+import hashlib
 import os
 import re
 import struct
+import subprocess
 
 import numpy as np
 import pytest
@@ -26,6 +28,28 @@ def test_library_exports_every_declared_symbol():
     for name in sorted(declared):
         assert hasattr(lib, name), name
     assert _native.lib().gaans_abi_version() == _native.ABI_VERSION
+
+
+# the exported names of an interface version (sha256 of the sorted names)
+EXPORTS = {14: "6011d4a77309168a", 15: "d3c9a16d34e7711d"}
+
+
+def test_exports_belong_to_the_interface_version():
+    header = open(os.path.join(REPO, "include", "gaans_w64.h")).read()
+    names = sorted(set(re.findall(r"^(?:int|const char\*)\s+(gaans_\w+)\(", header, re.M)))
+    digest = hashlib.sha256(" ".join(names).encode()).hexdigest()[:16]
+    assert EXPORTS[_native.ABI_VERSION] == digest, "new exports need a new version"
+
+
+def test_library_of_another_version_is_refused(tmp_path, monkeypatch):
+    from fast_compressai.coders.errors import CoderDependencyError
+    src, lib = tmp_path / "old.c", tmp_path / "old.so"  # as built before the newest entry points
+    src.write_text("int gaans_abi_version(void) { return %d; }" % (_native.ABI_VERSION - 1))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "library_path", lambda: str(lib))
+    with pytest.raises(CoderDependencyError, match="version mismatch"):
+        _native.lib()
 
 
 def test_host_selftest_division_constants():
