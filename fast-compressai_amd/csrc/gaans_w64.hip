@@ -3828,11 +3828,15 @@ struct EncPlan {
 // a smaller ring only flushes more often, a smaller block doubles the
 // per-block work (the batch-64 uniform workload's 16 staged tables of 255
 // symbols fit next to 8-step blocks with a 1024-word ring).
+// wg_regs[sb / 8]: the workgroups per CU that the registers of the kernel with
+// sb-step blocks and four mappers allow.  A plan that lets the whole grid be
+// resident at once (units without tickets, see encode_prepare) counts on no more.
 EncPlan plan_encode(const gaans_tables* t, int64_t P, int64_t units, const DevLds& d,
-                    int64_t extra = 0, bool range_ok = true,
+                    const int wg_regs[3], int64_t extra = 0, bool range_ok = true,
                     bool allow16 = false) {
   for (int64_t occ = occ_target(units, d, 4); occ >= 1; --occ)
-    for (int sb = allow16 ? 16 : 8; sb >= 4; sb >>= 1)
+    for (int sb = allow16 ? 16 : 8; sb >= 4; sb >>= 1) {
+      if (occ > wg_regs[sb / 8] && units <= occ * d.cus) continue;
       for (int ring = kRingWords; ring >= 2 * sb * kLanes && ring >= 1024; ring >>= 1) {
         Stage s;
         // + 2 entries: the staged copy starts at an even entry and ends on a
@@ -3843,6 +3847,7 @@ EncPlan plan_encode(const gaans_tables* t, int64_t P, int64_t units, const DevLd
                          (size_t)(fixed + 16 * (int64_t)s.nt_cap + 8 * (int64_t)s.ne_cap), occ,
                          ring};
       }
+    }
   // no tables staged (they read through L1/L2): the largest block allowed
   const int sb = allow16 ? 16 : 8;
   return EncPlan{Stage{0, 0, 0, 0}, sb, (size_t)enc_fixed_lds(sb, kRingWords), 1, kRingWords};
@@ -3960,6 +3965,29 @@ int allow_lds(const void* kernel, size_t bytes, const DevLds& d) {
   if (n_done < 64) {
     done_fn[n_done] = kernel;
     done_dev[n_done++] = d.dev;
+  }
+  return GAANS_OK;
+}
+
+// Workgroups of `threads` that a CU's registers and wave slots hold, as the
+// runtime counts them (asked once per kernel and device; the LDS is the plan's).
+int regs_residency(const void* kernel, int threads, const DevLds& d, int* out) {
+  static std::mutex mu;
+  static const void* known_fn[64];
+  static int known_dev[64], known[64];
+  static int n_known = 0;
+  std::lock_guard<std::mutex> g(mu);
+  for (int i = 0; i < n_known; ++i)
+    if (known_fn[i] == kernel && known_dev[i] == d.dev) {
+      *out = known[i];
+      return GAANS_OK;
+    }
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(out, kernel, threads, 0) != hipSuccess)
+    return fail(GAANS_EHIP, "cannot query a kernel's residency");
+  if (n_known < 64) {
+    known_fn[n_known] = kernel;
+    known_dev[n_known] = d.dev;
+    known[n_known++] = *out;
   }
   return GAANS_OK;
 }
@@ -4114,7 +4142,12 @@ int encode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
   // the coder waited about 135 of its 350 cycles per step at the barriers
   // (mean-scale hyperprior y, P = 4 and 16), and 16-step blocks give each
   // mapper wave two steps per block to overlap.
-  const EncPlan plan = plan_encode(tables, L.P, L.U, dl, extra, !gauss,
+  int wg_regs[3];  // by sb / 8: 4-, 8- and 16-step blocks
+  for (int i = 0; i < 3; ++i)
+    if ((rc = regs_residency(reinterpret_cast<const void*>(enc_kernel(mode, implicit, 4 << i, 4)),
+                             5 * kLanes, dl, &wg_regs[i])))
+      return rc;
+  const EncPlan plan = plan_encode(tables, L.P, L.U, dl, wg_regs, extra, !gauss,
                                    long_units || gauss);
   const Stage& st = plan.st;
   size_t lds = plan.lds + (size_t)extra;
@@ -4158,7 +4191,7 @@ int encode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
   a.stage_all = st.stage_all;
   a.ring_mask = (uint32_t)(plan.ring - 1);
   // fused encode: unit numbers from tickets unless the grid fits the device
-  // in one round at the plan's workgroups per CU
+  // in one round at the plan's workgroups per CU (which LDS and registers hold)
   a.ticket = L.U > plan.occ * (int64_t)dl.cus ? 1u : 0u;
   a.elect = L.U > (int64_t)dl.cus ? 1u : 0u;
   a.lds_bytes = (uint32_t)lds;
@@ -4892,6 +4925,23 @@ int gaans_run_decode_call(const gaans_decode_call* c) {
   if (!c) return fail(GAANS_EINVAL, "call pointer is NULL");
   return gaans_run_decode(c->plan, c->stream, c->payload_dev, c->payload_bytes, c->in[0],
                           c->in[1], c->in[2], c->out_dev, c->ctrl_dev, c->status_host);
+}
+
+int gaans_debug_plan(const gaans_plan* plan, int64_t out[3]) {
+  const EncPlanRec* r = reinterpret_cast<const EncPlanRec*>(plan);
+  if (!r || !out || r->h.magic != kPlanEncMagic)
+    return fail(GAANS_EINVAL, "not an encode plan (gaans_plan_encode)");
+  DevLds dl;
+  int rc, per_cu = 0;
+  if ((rc = plan_device(r->h)) || (rc = device_lds(&dl))) return rc;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &per_cu, reinterpret_cast<const void*>(r->e.kernel), (int)r->e.block, r->e.lds) !=
+      hipSuccess)
+    return fail(GAANS_EHIP, "cannot query a kernel's residency");
+  out[0] = r->e.grid;
+  out[1] = (int64_t)per_cu * dl.cus;
+  out[2] = r->e.a.ticket;
+  return GAANS_OK;
 }
 
 int gaans_debug_phases(void* buffer_dev, int64_t units, int32_t* wall_clock_khz) {

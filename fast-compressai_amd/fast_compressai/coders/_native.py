@@ -15,7 +15,7 @@ import threading
 from .errors import CoderDependencyError
 
 LIB_NAME = "libgaans_w64.so"
-ABI_VERSION = 15
+ABI_VERSION = 16
 CTRL_BYTES = 256
 PLAN_BYTES = 1536  # GAANS_PLAN_BYTES
 PHASE_SLOTS = 16  # GAANS_PHASE_SLOTS
@@ -148,6 +148,7 @@ def _declare(L) -> None:
                                      ctypes.c_int),
         "gaans_wait_host_word": ([p, p], ctypes.c_int),
         "gaans_debug_phases": ([p, i64, ctypes.POINTER(ctypes.c_int32)], ctypes.c_int),
+        "gaans_debug_plan": ([p, ctypes.POINTER(ctypes.c_int64)], ctypes.c_int),
         # plans are passed by address (c_void_p): no byref object per call
         "gaans_plan_encode": ([T, i32, i32, i32, f32, i64, i64, i64, i64, i32, p], ctypes.c_int),
         "gaans_plan_decode": ([T, i32, i32, i32, f32, i64, i64, i64, i64, i32, p], ctypes.c_int),

@@ -62,7 +62,7 @@
 extern "C" {
 #endif
 
-#define GAANS_ABI_VERSION 15
+#define GAANS_ABI_VERSION 16
 #define GAANS_CTRL_BYTES 256
 
 /* return codes */
@@ -499,6 +499,14 @@ int gaans_run_decode_call(const gaans_decode_call* call);
  * counter's rate on the current device.  No counterpart in the reference. */
 #define GAANS_PHASE_SLOTS 16
 int gaans_debug_phases(void* buffer_dev, int64_t units, int32_t* wall_clock_khz);
+
+/* What an encode plan counts on (for tests): out[0] its workgroups, out[1] how
+ * many of them the plan's device holds at once as the HIP runtime counts
+ * registers, wave slots and LDS, out[2] 1 if units take their numbers from the
+ * ticket counter.  Without tickets a unit is the workgroup index and may wait
+ * on any lower one, so the whole grid has to be resident: out[0] <= out[1].
+ * No counterpart in the reference. */
+int gaans_debug_plan(const gaans_plan* plan, int64_t out[3]);
 
 /* ---- host self test ------------------------------------------------------- */
 
