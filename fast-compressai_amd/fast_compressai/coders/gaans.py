@@ -39,6 +39,19 @@ CLONE_SLACK_BYTES = 32 << 20  # keep a view of the worst-case buffer below this 
 MAX_SLOTS = 8  # pinned word sets kept per stream (32 bytes each)
 
 
+class _Words:
+    """Four pinned 64-bit words.  The host clears and reads them through the
+    numpy view: a tensor made under ``torch.inference_mode`` refuses torch's own
+    in-place operations once it has ended (and the view is the faster one)."""
+
+    __slots__ = ("tensor", "view", "ptr")
+
+    def __init__(self) -> None:
+        self.tensor = torch.empty(4, dtype=torch.int64, pin_memory=True)
+        self.view = self.tensor.numpy()
+        self.ptr = self.tensor.data_ptr()
+
+
 class _StreamState:
     def __init__(self, device: torch.device) -> None:
         self.ctrl = torch.zeros(_native.CTRL_BYTES, dtype=torch.uint8, device=device)
@@ -56,17 +69,14 @@ class _StreamState:
         self.lock = threading.Lock()
         self.slots: list = []  # pinned words of calls in flight, returned when they end
 
-    def slot(self) -> torch.Tensor:
+    def slot(self) -> "_Words":
         """Pinned completion words for a call that is waited for later (the
-        caller holds ``lock``; ``give_back`` afterwards).  Cleared through the
-        host view: words made under ``torch.inference_mode`` refuse torch's own
-        in-place operations once it has ended."""
-        slot = self.slots.pop() if self.slots else torch.empty(4, dtype=torch.int64,
-                                                               pin_memory=True)
-        slot.numpy()[:] = 0
+        caller holds ``lock``; ``give_back`` afterwards)."""
+        slot = self.slots.pop() if self.slots else _Words()
+        slot.view.fill(0)
         return slot
 
-    def give_back(self, slot: torch.Tensor) -> None:
+    def give_back(self, slot: "_Words") -> None:
         with self.lock:
             if len(self.slots) < MAX_SLOTS:
                 self.slots.append(slot)
@@ -461,14 +471,14 @@ class _Pending:
     come.  ``finish`` waits for it and must be called once, whatever else
     happens in between: the word's memory is the call's until then."""
 
-    def __init__(self, st: _StreamState, stream_ptr: int, slot: torch.Tensor, word: int,
+    def __init__(self, st: _StreamState, stream_ptr: int, slot: _Words, word: int,
                  result) -> None:
         self._st, self._sp, self._slot, self._word, self._result = st, stream_ptr, slot, word, result
 
     def finish(self):
         _native.check(_native.lib().gaans_wait_host_word(
-            self._sp, self._slot.data_ptr() + self._word), "GA-ANS wait")
-        words = self._slot.tolist()
+            self._sp, self._slot.ptr + self._word), "GA-ANS wait")
+        words = self._slot.view.tolist()
         self._st.give_back(self._slot)
         return self._result(words)
 
@@ -492,7 +502,7 @@ def encode_latents_begin(tables: PreparedTables, B: int, N: int, C: int, P: int,
             ws, slot = st.ws(lay.workspace_bytes), st.slot()
             rc = _native.lib().gaans_enqueue_encode_latents(
                 plan, sp, y.data_ptr(), medians.data_ptr(), None, _ptr(y_hat), ws.data_ptr(),
-                ws.numel(), st.ctrl_ptr, out.data_ptr(), lay.max_payload_bytes, slot.data_ptr())
+                ws.numel(), st.ctrl_ptr, out.data_ptr(), lay.max_payload_bytes, slot.ptr)
         if rc:
             _native.check(rc, "GA-ANS encode")
     finally:
@@ -527,7 +537,7 @@ def decode_latents_begin(packed: torch.Tensor, tables: PreparedTables, B: int, N
             slot = st.slot()
             rc = _native.lib().gaans_enqueue_decode(plan, sp, packed.data_ptr(), packed.numel(),
                                                     medians.data_ptr(), None, None,
-                                                    out.data_ptr(), st.ctrl_ptr, slot.data_ptr())
+                                                    out.data_ptr(), st.ctrl_ptr, slot.ptr)
         if rc:
             _native.check(rc, "GA-ANS decode")
     finally:
