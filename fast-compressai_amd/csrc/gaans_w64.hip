@@ -219,8 +219,8 @@ __device__ __forceinline__ uint64_t ballot(bool pred) { return __builtin_amdgcn_
 // Keep a wave-uniform value in a scalar register.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// LDS at byte address a.  The kernels that use it have no static LDS, so their
-// dynamic LDS starts at address 0 and a byte offset in it is its address; a
+// LDS at byte address a.  The kernels that use it have no static LDS (a test
+// reads it from the built library), so their dynamic LDS starts at address 0 and a byte offset in it is its address; a
 // pointer made from the offset saves the add of that base (a constant 0 that
 // the compiler only learns after it has chosen the instructions).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -818,10 +818,11 @@ __device__ __forceinline__ void enc_records(const EncArgs& a, const Tabs& tb, in
 // the same records as enc_records, with the escape split computed only for
 // the steps that have an escaping lane.  With such offsets, sym - offset
 // wraps only to values of at least 65536, so (uint32)(sym - offset) <
-// nsym - 1 tests "ordinary" alone.  Returns false, having changed nothing,
-// when a lane of the block has an index outside the staged tables or a value
-// outside int32 (the caller then maps the block with enc_records); else sets
-// bit e of esc_steps for each step e with an escape.
+// nsym - 1 tests "ordinary" alone.  Returns false when a lane of the block has an
+// index outside the staged tables or a value outside int32: the caller then maps
+// the block with enc_records, which writes again what was written by then (only
+// the block's values at yh); else sets bit e of esc_steps for each step e with an
+// escape.
 //   z = enc_shift: the bits of freq - 1, entry word 0's high half: 16 less the
 //       word's leading zeros, and 0 for freq = 1, whose word has at least 16
 //       (none set, start = 0: 0xffffffff)
@@ -946,6 +947,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <int NS, bool kScalar, bool kKeep>
 __device__ __forceinline__ void enc_steps(uint32_t rec, uint32_t spare, uint32_t mask, uint32_t& x,
                                           uint32_t& n, int& wp, uint32_t* kz, uint32_t* kw) {
+  static_assert(NS != 2, "the first of two steps would have neither the read nor the store");
   __attribute__((address_space(3))) u32x4* recs = lds_ptr<u32x4>(rec);
   u32x4 r1 = recs[(NS - 1) * kLanes], r2 = r1;
   if (NS > 1) r2 = recs[(NS - 2) * kLanes];
@@ -965,7 +967,7 @@ __device__ __forceinline__ void enc_steps(uint32_t rec, uint32_t spare, uint32_t
     if (k >= 2) r2 = recs[(k - 2) * kLanes];
     if (k < NS - 1) *lds_ptr<uint16_t>(at0) = (uint16_t)x0;
     __builtin_amdgcn_sched_barrier(0);
-    if (NS == 1 || (NS == 2 && k == 1)) asm volatile("s_nop 0" : "+s"(m));  // neither of the two
+    if (NS == 1) asm volatile("s_nop 0" : "+s"(m));  // neither of the two
     uint32_t y, q, b, at, xn;
     if constexpr (kScalar) {
       wp -= __popcll(m);
@@ -3810,8 +3812,9 @@ bool fit_stage(const gaans_tables* t, int64_t P, int64_t per_table, int64_t per_
   return false;
 }
 
-// Encoder: metadata and both entry words per symbol; 8-step blocks, else
-// 4-step blocks (half the records) for each workgroups-per-CU count.
+// Encoder: metadata and both entry words per symbol; for each workgroups-per-CU
+// count 16-step blocks where the caller allows them, else 8-, else 4-step ones
+// (half the records each).
 struct EncPlan {
   Stage st;
   int sb;

@@ -52,6 +52,18 @@ def test_library_of_another_version_is_refused(tmp_path, monkeypatch):
         _native.lib()
 
 
+def test_coding_kernels_have_no_static_lds():
+    # they address LDS by byte offset, from 0: the code object's metadata, keys in
+    # alphabetical order (a small msgpack integer is its own byte)
+    data = open(_native.library_path(), "rb").read()
+    kernels = re.findall(rb"\.group_segment_fixed_size(.).{0,4000}?\.name(?:\xd9.|[\xa0-\xbf])(_Z\w+)",
+                         data, re.S)
+    coding = [(name, size) for size, name in kernels
+              if b"k_encode" in name or b"k_decode" in name]
+    assert len(coding) >= 60
+    assert all(size == b"\0" for _, size in coding), coding
+
+
 def test_host_selftest_division_constants():
     assert _native.lib().gaans_host_selftest() == 0, _native.last_error()
 
