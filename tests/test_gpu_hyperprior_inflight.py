@@ -15,8 +15,8 @@ from hyperprior_stub import make_hyperprior
 pytestmark = pytest.mark.gpu
 
 
-# one lane; less than a step; whole steps; a ragged last step; 16-step blocks
-# (12 units) and a chunk of several units.  Every 7th value lies outside its
+# one lane; less than a step; whole steps; a ragged last step in chunks of two
+# units; 16-step blocks (2 units of 384 and 192 steps).  Every 7th value lies outside its
 # table (an escape), the last one far outside.
 @pytest.mark.parametrize("shape,p_ch,segments", [
     ((1, 1, 1, 1), 1, 1), ((2, 3, 5, 7), 2, 1), ((1, 8, 8, 16), 4, 1), ((3, 6, 11, 13), 5, 2),
@@ -46,42 +46,62 @@ def test_encode_writes_the_dequantized_latents(gpu_device, shape, p_ch, segments
     assert enc.packed.cpu().numpy().tobytes() == ref
 
 
-@pytest.mark.parametrize("h_s_fails", [False, True])
-def test_error_of_z_is_raised_first(gpu_device, h_s_fails):
+def changed(payload, at, device):
+    blob = bytearray(payload.to_bytes())
+    blob[at] ^= 0x55
+    return WarpDivPayload._from_encoder(
+        packed=torch.frombuffer(blob, dtype=torch.uint8).to(device),
+        header_bytes=payload.header_bytes, chunk_len=payload.chunk_len,
+        p_ch=payload.p_ch, batch=payload.batch,
+        symbols_per_batch=payload.symbols_per_batch, cdf_count=payload.cdf_count,
+        coding_fingerprint=payload.coding_fingerprint, channels=payload.channels,
+        segments=payload.segments)
+
+
+def error_of(call, kind=CoderInputError):
+    with pytest.raises(kind) as e:
+        call()
+    return str(e.value)
+
+
+# what fails besides z: nothing of its own (y sees the z_hat of a failed z), h_s,
+# or y with another error than z's
+@pytest.mark.parametrize("also", ["nothing", "h_s", "y"])
+def test_error_of_z_is_raised_first(gpu_device, also):
     model = make_hyperprior(mean_scale=True).to(gpu_device)
     x = torch.rand(1, 3, 64, 64, device=gpu_device)
     fast = fast_compressai.accelerate(model, P=4, device=str(gpu_device))
     out = fast.compress(x)
-    good = fast.decompress(out["strings"], out["shape"])["x_hat"]
+    shape = out["shape"]
+    good = fast.decompress(out["strings"], shape)["x_hat"]
     y_payload, z_payload = out["strings"]
-    blob = bytearray(z_payload.to_bytes())
-    blob[-1] ^= 0x55  # the last unit's words: its final state no longer fits
-    bad = WarpDivPayload._from_encoder(
-        packed=torch.frombuffer(blob, dtype=torch.uint8).to(gpu_device),
-        header_bytes=z_payload.header_bytes, chunk_len=z_payload.chunk_len,
-        p_ch=z_payload.p_ch, batch=z_payload.batch,
-        symbols_per_batch=z_payload.symbols_per_batch, cdf_count=z_payload.cdf_count,
-        coding_fingerprint=z_payload.coding_fingerprint, channels=z_payload.channels,
-        segments=z_payload.segments)
+    # the last unit's words: its final state no longer fits
+    bad_z = changed(z_payload, -1, gpu_device)
     codec = fast._coder
     latents = codec.analyze(x)
-    nan_z = (latents[0], torch.full_like(latents[1], float("nan")))
-    params = codec._params
-    if h_s_fails:
+    nan_z = torch.full_like(latents[1], float("nan"))
+    z_decode = error_of(lambda: codec._z_decode(bad_z, shape)[0]())
+    z_encode = error_of(lambda: codec._z_encode(nan_z)[0]())
+    params, p_ch = codec._params, codec.p_ch
+    y = y_payload
+    print("case: z fails, and", also, flush=True)
+    if also == "h_s":
         def fail(z_hat):
             raise RuntimeError("h_s")
         codec._params = fail
-        with pytest.raises(RuntimeError, match="h_s"):
-            codec.encode_latents(latents)
-    print("case: z fails", h_s_fails, flush=True)
-    with pytest.raises(CoderInputError):
-        fast.decompress([y_payload, bad], out["shape"])
-    with pytest.raises(CoderInputError):
-        codec.encode_latents(nan_z)
-    codec._params = params
+        assert error_of(lambda: codec.encode_latents(latents), RuntimeError) == "h_s"
+    elif also == "y":
+        y = changed(y_payload, 0, gpu_device)  # the header's magic number
+        assert error_of(lambda: fast.decompress([y, z_payload], shape)) != z_decode
+    assert error_of(lambda: codec.decode_latents([y, bad_z], shape)) == z_decode
+    if also == "y":
+        codec.p_ch = latents[0].size(1) + 1  # z's is at most its own channel count
+        assert error_of(lambda: codec.encode_latents(latents)) != z_encode
+    assert error_of(lambda: codec.encode_latents((latents[0], nan_z))) == z_encode
+    codec._params, codec.p_ch = params, p_ch
     again = fast.compress(x)["strings"]
     assert [p.to_bytes() for p in again] == [p.to_bytes() for p in out["strings"]]
-    assert torch.equal(fast.decompress(out["strings"], out["shape"])["x_hat"], good)
+    assert torch.equal(fast.decompress(out["strings"], shape)["x_hat"], good)
 
 
 def test_calls_in_and_out_of_inference_mode(gpu_device):
