@@ -63,10 +63,10 @@ namespace {
 #endif
 constexpr int kMappers = GAANS_MAPPERS;  // mapper waves per decode workgroup
 // Encode workgroups: a coder wave and 4 mapper waves when several
-// workgroups share a CU, 8 when each has a CU to itself (the mappers are the
-// encoder's slower half: 8 take the 2160x3840 latent from 456 to 446 us and
-// the hyperprior y at P=16 from 91 to 68 us, while at three workgroups per
-// CU 8 cost more than they bring)
+// workgroups share a CU, 8 when each has a CU to itself: the mappers are then the
+// encoder's slower half (calls with 4 and 8: 2160x3840 latents, P = 8, 115.7 and
+// 105.9 us; 512x768 hyperprior, P = 16, 119.9 and 110.0; 512x768 symbols, P = 4,
+// 30.8 and 30.1)
 constexpr int kEncMaxWaves = 9;
 
 // per-wave hash, status and escape nibbles, then the escape count, the unit's
@@ -2870,6 +2870,15 @@ __device__ __forceinline__ void dec_block_search(const Tabs& tb, uint32_t rec, u
 // measurement build allows 5, since its phase points would otherwise push
 // the 16-step kernels past the 80 registers of 6 waves into scratch (its
 // phase times at three workgroups per CU are therefore approximate).
+// At 80 registers the Gaussian 16-step kernels keep a few words in scratch: the
+// coder's initial state, written before the tables are staged and read back as
+// the steps begin (8 bytes a lane, with the search lookups that is all), and with
+// the bucket lookups six constants of the mappers' path for a block with idle
+// lanes or unstaged tables (32 bytes); no full block touches them.  Without scratch
+// they were slower: built for 5 waves the third workgroup no longer fits on a CU
+// (64 x 192 x 32 x 48, six tables, P = 16: call 190.9 -> 228.1 us), and with the
+// scale search's eight coarse values in scalar registers the hyperprior y of
+// 512x768 at P = 16 decodes in 123.5 instead of 121.5 us (call).
 #ifdef GAANS_PHASE_TIMES
 constexpr int kDecWavesPerSimd = 5;
 #else
@@ -4133,11 +4142,12 @@ int encode_prepare(int mode, bool implicit, int32_t n_scales, float scale_bound,
   // the scale table, padded (stage_scales), at a 16-byte aligned offset
   const int64_t extra =
       mode == kModeGaussian ? align_up(4 * ((int64_t)n_scales + kGaussPad), 16) + 16 : 0;
-  // 16-step blocks for long units only (the coder waits for the first
-  // block to be mapped, so short units lose more than the per-block saving
-  // gains: slower at 96 steps; at 384 steps 1x192x32x48, P = 16, 38.9 -> 33.8
-  // us and the batch-64 skew draw 49.8 -> 44.5 us; at 1,020 steps the
-  // 2160x3840 latent 94 -> 80 us)
+  // 16-step blocks for long units only: the coder waits for the first block to
+  // be mapped, which a short unit does not make up for.  Calls with 8- and 16-step
+  // blocks, 192 channels of 32 x 64 symbols, one image and 48 of 96 channels: at
+  // 256 steps a unit 41.3 and 37.8 us, 57.2 and 53.2; at 192 steps 36.6 and 34.9,
+  // 52.3 and 50.7; at 96 steps (512x768, P = 4) no difference beyond the noise.
+  // The line lies where the gain is clear; it could lie lower.
   const bool long_units = L.seg_cap >= 256 * kLanes;
   const bool gauss = mode == kModeGaussian;
   if (gauss) implicit = false;

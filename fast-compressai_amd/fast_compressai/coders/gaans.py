@@ -5,9 +5,12 @@ once; every launch leaves it zeroed), a reusable workspace (zeroed when it
 is allocated: the fused encode's look-back words must start at zero, and
 every launch leaves them so), and two small pinned host buffers that the
 kernels write the payload size / status into, and a completion word that
-carries both.  The device orders calls on one stream; the pinned words are
-also shared by the host threads that call on that stream, so a lock per
-(device, stream) is held from a call's launch until its words are read.
+carries both.  The device orders calls on one stream, which is what protects
+the workspace and the control block; the pinned words are also shared by the
+host threads that call on that stream, so a lock per (device, stream) is held
+from a call's launch until its words are read.  Calls that are waited for later
+(``*_begin``) hold it around the launch only and have pinned words of their own
+until they are finished (``_StreamState.slot``).
 
 Each shape gets a call plan (``gaans_plan_encode`` / ``gaans_plan_decode``:
 layout, LDS plan, kernel variant and argument block, computed once and kept
