@@ -116,7 +116,8 @@ class HyperpriorWarpDivCodec:
     # share of h_s and y.  With z_hat written by the encode kernel instead of five
     # elementwise launches, a 512x768 image at P = 16 went from 145.7 to 112.5 us
     # (encode) and from 156.9 to 121.9 us (decode), h_s itself not counted.  z's
-    # error is still the one raised when both fail.
+    # error is still the one raised when both fail; until then h_s and y run on
+    # what a bad z left in z_hat.
     def _z_encode(self, z: torch.Tensor):
         """Enqueue z's encode; returns (finish -> payload, z_hat)."""
         eb = self.model.entropy_bottleneck

@@ -1,6 +1,8 @@
 """z of the hyperpriors coded without a wait before ``h_s`` and y: z_hat as the
 encode kernel writes it, and whose error is raised when z and y both fail."""
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -44,6 +46,18 @@ def test_encode_writes_the_dequantized_latents(gpu_device, shape, p_ch, segments
     sym = np.rint(y - med[None, :, None]).astype(np.int64).astype(np.int32).reshape(B, -1)
     ref = O.gaans_encode(sym, w.indexes, w.cdfs, w.cdf_sizes, w.offsets, p_ch, None, segments)
     assert enc.packed.cpu().numpy().tobytes() == ref
+
+
+def test_strided_z(gpu_device):
+    model = make_hyperprior(mean_scale=True).to(gpu_device)
+    codec = fast_compressai.accelerate(model, P=4, device=str(gpu_device))._coder
+    z = torch.randn(2, 8, 5, 7, device=gpu_device) * 3
+    print("case: strided z", flush=True)
+    with torch.no_grad():
+        finish, z_hat = codec._z_encode(z)
+        finish_s, z_hat_s = codec._z_encode(z.contiguous(memory_format=torch.channels_last))
+    assert finish().to_bytes() == finish_s().to_bytes()
+    assert torch.equal(z_hat, z_hat_s) and z_hat_s.stride() != z_hat.stride()
 
 
 def changed(payload, at, device):
@@ -117,3 +131,42 @@ def test_calls_in_and_out_of_inference_mode(gpu_device):
             y_hat = codec.decode_latents(out["strings"], out["shape"])
             got.append([p.to_bytes() for p in out["strings"]] + [y_hat.cpu().numpy().tobytes()])
     assert got[0] == got[1] == got[2]
+
+
+# two host threads on the default stream and two on streams of their own, z of
+# each in flight while its y, or another thread's z, is enqueued
+def test_threads_and_streams(gpu_device):
+    model = make_hyperprior(mean_scale=True).to(gpu_device)
+    codec = fast_compressai.accelerate(model, P=4, device=str(gpu_device))._coder
+    with torch.no_grad():
+        latents = [codec.analyze(torch.rand(1 + i % 2, 3, 64, 64 << i % 2, device=gpu_device))
+                   for i in range(4)]
+    want = []
+    for pair in latents:
+        out = codec.encode_latents(pair)
+        want.append([p.to_bytes() for p in out["strings"]]
+                    + [codec.decode_latents(out["strings"], out["shape"]).cpu()])
+    torch.cuda.synchronize()
+    streams = [torch.cuda.current_stream(gpu_device)] * 2 + [torch.cuda.Stream(gpu_device)
+                                                             for _ in range(2)]
+    wrong = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(streams[i]):
+                for _ in range(20):
+                    out = codec.encode_latents(latents[i])
+                    y_hat = codec.decode_latents(out["strings"], out["shape"]).cpu()
+                    got = [p.to_bytes() for p in out["strings"]]
+                    if got != want[i][:2] or not torch.equal(y_hat, want[i][2]):
+                        wrong.append((i, "other results"))
+        except Exception as e:  # shown by the assertion below
+            wrong.append((i, repr(e)))
+
+    print("case: threads and streams", flush=True)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
